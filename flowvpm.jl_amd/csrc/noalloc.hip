@@ -4,7 +4,7 @@
 // hipMalloc on first use.  Callers that cannot allocate (code under HIP graph
 // capture, tight serving loops, harnesses that forbid it) call
 // vpm_uj_direct_noalloc instead: the same kernels, with every scratch buffer
-// (Morton keys and permutation, the radix sort's temp storage, the staged
+// (sort keys and permutation, the radix sort's temp storage, the staged
 // sources, the K x 14 (or 12) FP64 partial sums per target) taken from one
 // file-scope device array of kNoAllocBytes.  Each GPU holds its own copy of
 // the array until the process ends; its address on a device is looked up

@@ -281,7 +281,7 @@ __device__ __forceinline__ void tile_f32c(int n, const float4* lpos, const float
     for (int g = 0; g < NG; ++g) {
         uint64_t fb = far[g];
         if (fb == ~0ull) {
-            // the whole group is far (the common case in Morton order): a
+            // the whole group is far (the common case in sorted order): a
             // straight-line loop with immediate LDS offsets, no scalar
             // bookkeeping per source
 #pragma unroll 16

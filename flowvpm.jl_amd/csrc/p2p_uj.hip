@@ -10,7 +10,7 @@
 // F32C (FP32 pair arithmetic, compensated sums):
 //  * positions are differenced relative to the block origin O (the block's
 //    first target, FP64): t' = fl32(t - O), s' = fl32(s - O).  After a
-//    spatial (Morton) sort, |t'|,|s'| are small for every pair that matters,
+//    spatial (Hilbert-curve) sort, |t'|,|s'| are small for every pair that matters,
 //    so dx = t' - s' keeps FP32 relative accuracy of the distance itself
 //    rather than of the absolute coordinate;
 //  * with Gamma' = -Gamma/(4 pi) per source, a pair contributes
@@ -298,23 +298,51 @@ __device__ __forceinline__ uint64_t spread21(uint64_t v)
     return v;
 }
 
-__global__ __launch_bounds__(kBlock) void morton_kernel(const double* __restrict__ P, int64_t np,
-                                                        const double* __restrict__ bb,
-                                                        uint64_t* __restrict__ keys,
-                                                        uint32_t* __restrict__ iota)
+// Position along the 3-D Hilbert curve of 21 bits per axis (J. Skilling,
+// "Programming the Hilbert curve", AIP Conf. Proc. 707, 2004: the inverse
+// undo of the curve's rotations per bit, a Gray decode, then the bits of the
+// three axes interleaved).  Consecutive cells of this curve always share a
+// face, so every run of particles is compact; a Z-order run that crosses a
+// jump of its curve has a box of up to the whole domain, and all its pairs
+// then fail the box tests of the kernels (near/far split, tile skipping).
+__global__ __launch_bounds__(kBlock) void hilbert_kernel(const double* __restrict__ P, int64_t np,
+                                                         const double* __restrict__ bb,
+                                                         uint64_t* __restrict__ keys,
+                                                         uint32_t* __restrict__ iota)
 {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i >= np) return;
     const double ext = fmax(fmax(bb[3] - bb[0], bb[4] - bb[1]), fmax(bb[5] - bb[2], 1e-300));
     const double sc = 2097151.0 / ext;
-    uint64_t k = 0;
+    uint32_t x[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-        double u = (P[i * NF + RX + c] - bb[c]) * sc;
-        u = fmin(fmax(u, 0.0), 2097151.0);
-        k |= spread21((uint64_t)u) << c;
+        const double u = (P[i * NF + RX + c] - bb[c]) * sc;
+        x[c] = (uint32_t)fmin(fmax(u, 0.0), 2097151.0);
     }
-    keys[i] = k;
+    for (uint32_t q = 1u << 20; q > 1; q >>= 1) {
+        const uint32_t low = q - 1;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            if (x[c] & q) {
+                x[0] ^= low;               // invert the lower bits of axis 0
+            } else {
+                const uint32_t t = (x[0] ^ x[c]) & low;   // exchange them with axis c
+                x[0] ^= t;
+                x[c] ^= t;
+            }
+        }
+    }
+    x[1] ^= x[0];
+    x[2] ^= x[1];
+    uint32_t t = x[2];                     // prefix parity of axis 2 above each bit
+    t ^= t >> 1;
+    t ^= t >> 2;
+    t ^= t >> 4;
+    t ^= t >> 8;
+    t ^= t >> 16;
+    t >>= 1;
+    keys[i] = spread21(x[0] ^ t) << 2 | spread21(x[1] ^ t) << 1 | spread21(x[2] ^ t);
     iota[i] = (uint32_t)i;
 }
 
@@ -404,7 +432,7 @@ int sort_scratch_bytes(vpm_field f, size_t& bytes)
     return VPM_OK;
 }
 
-// Morton (Z-order) permutation of the field's particles: perm[k] is the
+// Hilbert-curve permutation of the field's particles: perm[k] is the
 // particle at sorted position k.  Reused until positions change (not when
 // it lives in an arena).
 int sort_field(vpm_field f, const uint32_t*& perm, Arena* ar)
@@ -429,9 +457,9 @@ int sort_field(vpm_field f, const uint32_t*& perm, Arena* ar)
     VPM_LAUNCH_CHECK("bbox_partial");
     hipLaunchKernelGGL(bbox_final_kernel, dim3(1), dim3(64), 0, f->stream, bb, kSortBoxes);
     VPM_LAUNCH_CHECK("bbox_final");
-    hipLaunchKernelGGL(morton_kernel, dim3(nblocks(np)), dim3(kBlock), 0, f->stream, f->P, np, bb,
+    hipLaunchKernelGGL(hilbert_kernel, dim3(nblocks(np)), dim3(kBlock), 0, f->stream, f->P, np, bb,
                        (uint64_t*)kp, (uint32_t*)ip);
-    VPM_LAUNCH_CHECK("morton");
+    VPM_LAUNCH_CHECK("hilbert");
     size_t tmp = 0;
     hipError_t e = rocprim::radix_sort_pairs(nullptr, tmp, (const uint64_t*)kp, (uint64_t*)k2p,
                                              (const uint32_t*)ip, (uint32_t*)pp, (unsigned)np, 0,

@@ -6,7 +6,7 @@
 // skip: the self term is Gamma_i zeta(0)/sigma_i^3).  The viscous scheme's
 // RBF reset evaluates the vorticity field through it.
 //
-// F32C: the U/J tiling (lanes own targets, sources through LDS, Morton
+// F32C: the U/J tiling (lanes own targets, sources through LDS, sorted
 // order, hi/lo positions relative to the block origin, per-tile TwoSum).
 // zeta_sigma is (a, b) per source as in E_str: b exp2(a r^2) (Gaussian-erf),
 // b exp2(a r^3) (Gaussian), b (1 + a r^2)^-3.5 (Winckelmans).  Sources whose
