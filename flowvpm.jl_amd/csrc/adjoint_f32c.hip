@@ -474,7 +474,9 @@ int launch_uj_adjoint_f32c(vpm_field f, int kernel, const double* dU, const doub
     const int64_t np = f->np;
     int rc;
     Staged S;
-    if ((rc = stage_field(f, kernel, VPM_PREC_F32C, true, S))) return rc;
+    // below 2^14 particles the runs are few and large in either order
+    const Order order = np >= (1 << 14) ? kHilbert : kZOrder;
+    if ((rc = stage_field(f, kernel, VPM_PREC_F32C, order, S))) return rc;
     const unsigned nb = (unsigned)((np + kBlock - 1) / kBlock);
     hipLaunchKernelGGL(pack_adj_cot_kernel, dim3(nb), dim3(kBlock), 0, f->stream, dU, dJ, S.perm, np, tcot);
     hipError_t e = hipGetLastError();

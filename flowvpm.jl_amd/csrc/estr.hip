@@ -552,7 +552,7 @@ int launch_estr_f64far(vpm_field f, int kernel, int transposed)
     if (np == 0) return VPM_OK;
     int rc;
     const uint32_t* perm = nullptr;
-    if ((rc = sort_field(f, perm))) return rc;
+    if ((rc = sort_field(f, kZOrder, perm))) return rc;
     const int64_t ld = f->cap;
     const int64_t ntile = (np + kTile - 1) / kTile;
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };

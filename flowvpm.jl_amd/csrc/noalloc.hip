@@ -17,7 +17,7 @@
 #include <mutex>
 #include <string>
 
-#include "vpm_internal.h"
+#include "uj_far.h"
 
 namespace vpm {
 
@@ -61,7 +61,8 @@ size_t al(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Bytes of the array one evaluation takes with K source splits (the order of
 // stage_field, sort_field and launch_uj; every piece 256-byte aligned).
-static int noalloc_bytes(vpm_field f, int precision, bool sort, int64_t K, size_t& out)
+// With `far`, the far kernel's boxes, words and partial sums too.
+static int noalloc_bytes(vpm_field f, int precision, bool sort, int64_t K, bool far, size_t& out)
 {
     const size_t np = (size_t)f->np;
     if (precision == VPM_PREC_F64) {
@@ -71,8 +72,13 @@ static int noalloc_bytes(vpm_field f, int precision, bool sort, int64_t K, size_
     size_t sb = 0;
     if (sort && np > 1)
         if (int rc = sort_scratch_bytes(f, sb)) return rc;
-    out = al(sizeof(double) * 3 * np) + al(sizeof(float4) * np) + al(sizeof(float) * np) + sb +
-          al(sizeof(double) * kAccF32 * K * np);
+    out = al(sizeof(double) * 3 * np) + al(sizeof(float4) * np) + al(sizeof(float) * np) + sb;
+    if (far) {
+        const FarSplit k = far_split(f->np, f->np, K);
+        K = k.far + k.rest;
+        out += al(far_scratch_bytes(f->np, f->np));
+    }
+    out += al(sizeof(double) * kAccF32 * K * np);
     return VPM_OK;
 }
 
@@ -102,23 +108,24 @@ extern "C" int vpm_uj_direct_noalloc(vpm_field f, const vpm_config* cfg, uint32_
     // the splits vpm_uj_direct would take, fewer when they do not fit
     int64_t K = 1, chunk = 0;
     size_t need = 0;
+    bool far = false;
     if (np > 0) {
         choose_split(np, np, 0, K, chunk);
         size_t one = 0;
-        if ((rc = noalloc_bytes(f, cfg->precision, sort, 1, one))) return rc;
+        if ((rc = noalloc_bytes(f, cfg->precision, sort, 1, false, one))) return rc;
         if (one > kNoAllocBytes)
             return fail(VPM_ERANGE, "vpm_uj_direct_noalloc: " + std::to_string(np) + " particles need " +
                                         std::to_string(one) + " bytes of scratch, above the " +
                                         std::to_string(kNoAllocBytes) + "-byte maximum");
-        if ((rc = noalloc_bytes(f, cfg->precision, sort, K, need))) return rc;
-        if (need > kNoAllocBytes) {
-            const size_t per_split = sizeof(double) * (cfg->precision == VPM_PREC_F64 ? kAccF64 : kAccF32) *
-                                     (size_t)np;
-            K = std::min<int64_t>(K, 1 + (int64_t)((kNoAllocBytes - one) / al(per_split)));
-            if ((rc = noalloc_bytes(f, cfg->precision, sort, K, need))) return rc;
-            while (K > 1 && need > kNoAllocBytes)
-                if ((rc = noalloc_bytes(f, cfg->precision, sort, --K, need))) return rc;
+        // the far kernel where its scratch fits beside one split of each
+        far = sort && far_applies(cfg->kernel, cfg->precision, np, np) && far_batch(np, np) == np;
+        if (far) {
+            if ((rc = noalloc_bytes(f, cfg->precision, sort, 1, true, need))) return rc;
+            far = need <= kNoAllocBytes;
         }
+        if ((rc = noalloc_bytes(f, cfg->precision, sort, K, far, need))) return rc;
+        while (K > 1 && need > kNoAllocBytes)
+            if ((rc = noalloc_bytes(f, cfg->precision, sort, --K, far, need))) return rc;
     }
     DeviceScratch& d = g_dev[f->device];
     std::lock_guard<std::mutex> dlk(d.mu);
@@ -126,8 +133,8 @@ extern "C" int vpm_uj_direct_noalloc(vpm_field f, const vpm_config* cfg, uint32_
     if (flags & VPM_UJ_RESET) if ((rc = launch_reset(f, 0))) return rc;
     if (flags & VPM_UJ_RESET_SFS) if ((rc = launch_reset(f, 1))) return rc;
     Staged st;
-    if ((rc = stage_field(f, cfg->kernel, cfg->precision, sort, st, &ar)) ||
-        (rc = launch_uj(f, st, 0, np, st, 0, np, cfg->kernel, cfg->precision, &ar, K))) {
+    if ((rc = stage_field(f, cfg->kernel, cfg->precision, !sort ? kStorage : far ? kHilbert : kZOrder, st, &ar)) ||
+        (rc = launch_uj(f, st, 0, np, st, 0, np, cfg->kernel, cfg->precision, far, &ar, K))) {
         (void)hipStreamSynchronize(f->stream);   // no launch of this call still reads the array
         return rc;
     }

@@ -254,7 +254,7 @@ __device__ __forceinline__ void fold_u(float (&acc)[kAccF32], float (&sum)[kAccF
 // (then some lane may be near; the test is conservative).  The far and the
 // near sources are then visited by iterating over the set bits of the two
 // masks (scalar loop control), so the far loop body is straight-line.
-template <int K, int NG = kTile / 64>
+template <int K, int NG = kTile / 64, bool FOLD = (NG > 1)>
 __device__ __forceinline__ void tile_f32c(int n, const float4* lpos, const float4* lgs, const float4* llo,
                                           float tx, float ty, float tz, float tlx, float tly, float tlz,
                                           const WaveBox& box, float (&acc)[kAccF32], float (&sum)[kAccF32],
@@ -297,7 +297,7 @@ __device__ __forceinline__ void tile_f32c(int n, const float4* lpos, const float
     // Near pairs carry the largest terms of a sum that may cancel to far
     // below them, so over 256-source tiles the U partials are folded into
     // the TwoSum pairs every kNearFold near pairs (the count is
-    // wave-uniform).  One-group tiles (the wave-per-leaf list kernels) fold
+    // wave-uniform).  The wave-per-leaf list kernels (FOLD = false) fold
     // every 64 sources anyway.
     int nn = 0;
 #pragma unroll
@@ -307,7 +307,7 @@ __device__ __forceinline__ void tile_f32c(int n, const float4* lpos, const float
             const int s = g * 64 + __builtin_ctzll(nb);
             nb &= nb - 1;
             near_pair<K>(tx, ty, tz, tlx, tly, tlz, lpos[s], lgs[s], llo[s], acc);
-            if constexpr (NG > 1) {
+            if constexpr (FOLD) {
                 if (++nn == kNearFold) {
                     fold_u(acc, sum, err);
                     nn = 0;

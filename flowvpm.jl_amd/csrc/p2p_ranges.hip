@@ -553,7 +553,7 @@ int launch_p2p_plan(vpm_field f, int kernel, int precision, const DevPlan& dp)
 {
     if (dp.nitems == 0) return VPM_OK;
     Staged st;
-    if (int rc = stage_field(f, kernel, precision, false, st)) return rc;
+    if (int rc = stage_field(f, kernel, precision, kStorage, st)) return rc;
     const RangeItem* d_items = dp.items;
     const int2* d_src = dp.src;
     const dim3 grid((unsigned)dp.nitems);

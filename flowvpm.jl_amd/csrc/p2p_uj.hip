@@ -10,7 +10,7 @@
 // F32C (FP32 pair arithmetic, compensated sums):
 //  * positions are differenced relative to the block origin O (the block's
 //    first target, FP64): t' = fl32(t - O), s' = fl32(s - O).  After a
-//    spatial (Hilbert-curve) sort, |t'|,|s'| are small for every pair that matters,
+//    spatial sort (curve_kernel), |t'|,|s'| are small for every pair that matters,
 //    so dx = t' - s' keeps FP32 relative accuracy of the distance itself
 //    rather than of the absolute coordinate;
 //  * with Gamma' = -Gamma/(4 pi) per source, a pair contributes
@@ -36,6 +36,7 @@
 #include <rocprim/device/device_radix_sort.hpp>
 
 #include "p2p_pair.h"
+#include "uj_far.h"
 
 
 namespace vpm {
@@ -298,17 +299,21 @@ __device__ __forceinline__ uint64_t spread21(uint64_t v)
     return v;
 }
 
-// Position along the 3-D Hilbert curve of 21 bits per axis (J. Skilling,
-// "Programming the Hilbert curve", AIP Conf. Proc. 707, 2004: the inverse
-// undo of the curve's rotations per bit, a Gray decode, then the bits of the
-// three axes interleaved).  Consecutive cells of this curve always share a
-// face, so every run of particles is compact; a Z-order run that crosses a
-// jump of its curve has a box of up to the whole domain, and all its pairs
-// then fail the box tests of the kernels (near/far split, tile skipping).
-__global__ __launch_bounds__(kBlock) void hilbert_kernel(const double* __restrict__ P, int64_t np,
-                                                         const double* __restrict__ bb,
-                                                         uint64_t* __restrict__ keys,
-                                                         uint32_t* __restrict__ iota)
+// Position along a space-filling curve of 21 bits per axis: the Z-order curve,
+// or the 3-D Hilbert curve (J. Skilling, "Programming the Hilbert curve", AIP
+// Conf. Proc. 707, 2004: the inverse undo of the curve's rotations per bit, a
+// Gray decode, then the bits of the three axes interleaved).  Consecutive
+// cells of the Hilbert curve always share a face, so every run of particles is
+// compact; a Z-order run that crosses a jump of its curve has a box of up to
+// the whole domain, and all its pairs then fail the box tests of the kernels.
+// The far kernel and the adjoint take the Hilbert order: 1.0 % instead of 1.6 %
+// of the 2^20 jet's pairs are left to the VALU, 23 % of the 65,536 cloud's
+// U/J time and 5 % of the 32,768 cloud's adjoint.
+template <bool HILBERT>
+__global__ __launch_bounds__(kBlock) void curve_kernel(const double* __restrict__ P, int64_t np,
+                                                       const double* __restrict__ bb,
+                                                       uint64_t* __restrict__ keys,
+                                                       uint32_t* __restrict__ iota)
 {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i >= np) return;
@@ -319,6 +324,11 @@ __global__ __launch_bounds__(kBlock) void hilbert_kernel(const double* __restric
     for (int c = 0; c < 3; ++c) {
         const double u = (P[i * NF + RX + c] - bb[c]) * sc;
         x[c] = (uint32_t)fmin(fmax(u, 0.0), 2097151.0);
+    }
+    iota[i] = (uint32_t)i;
+    if constexpr (!HILBERT) {
+        keys[i] = spread21(x[0]) | spread21(x[1]) << 1 | spread21(x[2]) << 2;
+        return;
     }
     for (uint32_t q = 1u << 20; q > 1; q >>= 1) {
         const uint32_t low = q - 1;
@@ -343,7 +353,6 @@ __global__ __launch_bounds__(kBlock) void hilbert_kernel(const double* __restric
     t ^= t >> 16;
     t >>= 1;
     keys[i] = spread21(x[0] ^ t) << 2 | spread21(x[1] ^ t) << 1 | spread21(x[2] ^ t);
-    iota[i] = (uint32_t)i;
 }
 
 template <int K>
@@ -432,34 +441,36 @@ int sort_scratch_bytes(vpm_field f, size_t& bytes)
     return VPM_OK;
 }
 
-// Hilbert-curve permutation of the field's particles: perm[k] is the
+// Permutation of the field's particles along a curve: perm[k] is the
 // particle at sorted position k.  Reused until positions change (not when
 // it lives in an arena).
-int sort_field(vpm_field f, const uint32_t*& perm, Arena* ar)
+int sort_field(vpm_field f, Order order, const uint32_t*& perm, Arena* ar)
 {
     const int64_t np = f->np;
     const int64_t ld = ar ? np : f->cap;
     int rc;
     perm = nullptr;
-    if (np <= 1) return VPM_OK;
-    if (f->perm_valid && !ar) {
-        perm = (const uint32_t*)f->perm.p;
+    if (np <= 1 || order == kStorage) return VPM_OK;
+    const int c = order == kHilbert ? 1 : 0;
+    if (f->perm_valid[c] && !ar) {
+        perm = (const uint32_t*)f->perm[c].p;
         return VPM_OK;
     }
     void *bbp, *kp, *k2p, *pp, *ip;
     if ((rc = take_buffer(f, f->bbox, sizeof(double) * (6 + 6 * kSortBoxes), ar, bbp, "bbox"))) return rc;
     if ((rc = take_buffer(f, f->keys, sizeof(uint64_t) * (size_t)ld, ar, kp, "keys"))) return rc;
     if ((rc = take_buffer(f, f->keys2, sizeof(uint64_t) * (size_t)ld, ar, k2p, "keys"))) return rc;
-    if ((rc = take_buffer(f, f->perm, sizeof(uint32_t) * (size_t)ld, ar, pp, "perm"))) return rc;
+    if ((rc = take_buffer(f, f->perm[c], sizeof(uint32_t) * (size_t)ld, ar, pp, "perm"))) return rc;
     if ((rc = take_buffer(f, f->iota, sizeof(uint32_t) * (size_t)ld, ar, ip, "perm"))) return rc;
     double* bb = (double*)bbp;
     hipLaunchKernelGGL(bbox_partial_kernel, dim3(kSortBoxes), dim3(kBlock), 0, f->stream, f->P, np, bb);
     VPM_LAUNCH_CHECK("bbox_partial");
     hipLaunchKernelGGL(bbox_final_kernel, dim3(1), dim3(64), 0, f->stream, bb, kSortBoxes);
     VPM_LAUNCH_CHECK("bbox_final");
-    hipLaunchKernelGGL(hilbert_kernel, dim3(nblocks(np)), dim3(kBlock), 0, f->stream, f->P, np, bb,
-                       (uint64_t*)kp, (uint32_t*)ip);
-    VPM_LAUNCH_CHECK("hilbert");
+    const auto curve = c ? curve_kernel<true> : curve_kernel<false>;
+    hipLaunchKernelGGL(curve, dim3(nblocks(np)), dim3(kBlock), 0, f->stream, f->P, np, bb, (uint64_t*)kp,
+                       (uint32_t*)ip);
+    VPM_LAUNCH_CHECK("curve");
     size_t tmp = 0;
     hipError_t e = rocprim::radix_sort_pairs(nullptr, tmp, (const uint64_t*)kp, (uint64_t*)k2p,
                                              (const uint32_t*)ip, (uint32_t*)pp, (unsigned)np, 0,
@@ -471,12 +482,12 @@ int sort_field(vpm_field f, const uint32_t*& perm, Arena* ar)
                                   (const uint32_t*)ip, (uint32_t*)pp, (unsigned)np, 0, 63,
                                   f->stream);
     if (e != hipSuccess) return hip_fail(e, "radix_sort_pairs");
-    if (!ar) f->perm_valid = true;
+    if (!ar) f->perm_valid[c] = true;
     perm = (const uint32_t*)pp;
     return VPM_OK;
 }
 
-int stage_field(vpm_field f, int kernel, int precision, bool sort, Staged& out, Arena* ar)
+int stage_field(vpm_field f, int kernel, int precision, Order order, Staged& out, Arena* ar)
 {
     const int64_t np = f->np;
     const int64_t ld = ar ? np : f->cap;
@@ -498,7 +509,7 @@ int stage_field(vpm_field f, int kernel, int precision, bool sort, Staged& out, 
     if (precision == kPrecF64Far) {
         if ((rc = take_buffer(f, f->g64, sizeof(double4) * (size_t)ld, ar, gp, "sources"))) return rc;
         const uint32_t* perm = nullptr;
-        if (sort && np > 1 && (rc = sort_field(f, perm, ar))) return rc;
+        if ((rc = sort_field(f, order, perm, ar))) return rc;
         hipLaunchKernelGGL(pack_f64far_kernel, dim3(nblocks(np)), dim3(kBlock), 0, f->stream,
                            f->P, np, perm, (double*)posp, ld, (double4*)gp);
         VPM_LAUNCH_CHECK("pack_f64far");
@@ -509,7 +520,7 @@ int stage_field(vpm_field f, int kernel, int precision, bool sort, Staged& out, 
     if ((rc = take_buffer(f, f->gs, sizeof(float4) * (size_t)ld, ar, gp, "sources"))) return rc;
     if ((rc = take_buffer(f, f->cut, sizeof(float) * (size_t)ld, ar, cp, "sources"))) return rc;
     const uint32_t* perm = nullptr;
-    if (sort && np > 1 && (rc = sort_field(f, perm, ar))) return rc;
+    if ((rc = sort_field(f, order, perm, ar))) return rc;
     switch (kernel) {
 #define VPM_PACK(KID)                                                                                  \
     case KID:                                                                                          \
@@ -551,10 +562,37 @@ void choose_split(int64_t nt, int64_t ns, int64_t kmax, int64_t& K, int64_t& chu
     if (K < 1) K = 1;
 }
 
+// F32C launch split by the words of uj_far.hip: the far groups on the matrix
+// cores, the rest wave by wave on the VALU, in batches of targets.
+static int launch_uj_split(vpm_field ft, const Staged& T, int64_t nt, const Staged& S, int64_t ns, int kernel,
+                           Arena* ar, int64_t kmax)
+{
+    const int64_t bt = far_batch(nt, ns);
+    const FarSplit k = far_split(bt, ns, kmax);
+    int rc;
+    void *fp, *pp;
+    if ((rc = take_buffer(ft, ft->far, far_scratch_bytes(bt, ns), ar, fp, "far field"))) return rc;
+    const size_t bytes = sizeof(double) * kAccF32 * (size_t)(k.far + k.rest) * (size_t)bt;
+    if ((rc = take_buffer(ft, ft->part, bytes, ar, pp, "partial sums"))) return rc;
+    double* part = (double*)pp;
+    for (int64_t t0 = 0; t0 < nt; t0 += bt) {
+        const int64_t n = std::min(bt, nt - t0);
+        timing_begin(ft);
+        if ((rc = launch_uj_far(ft->stream, T, t0, n, S, ns, kernel, k, fp, part))) return rc;
+        timing_end(ft, 0);
+        hipLaunchKernelGGL(finalize_f32c_kernel, dim3(nblocks(n)), dim3(kBlock), 0, ft->stream, (const double*)part,
+                           n, (int)(k.far + k.rest), n, T.perm, t0, ft->P);
+        VPM_LAUNCH_CHECK("finalize_f32c");
+    }
+    return VPM_OK;
+}
+
 int launch_uj(vpm_field ft, const Staged& T, int64_t t0, int64_t nt, const Staged& S, int64_t s0,
-              int64_t s1, int kernel, int precision, Arena* ar, int64_t kmax)
+              int64_t s1, int kernel, int precision, bool far, Arena* ar, int64_t kmax)
 {
     if (nt <= 0 || s1 <= s0) return VPM_OK;
+    if (far && t0 == 0 && s0 == 0 && far_applies(kernel, precision, nt, s1))
+        return launch_uj_split(ft, T, nt, S, s1, kernel, ar, kmax);
     int64_t K, chunk;
     choose_split(nt, s1 - s0, kmax, K, chunk);
     const int acc = precision == VPM_PREC_F64 ? kAccF64 : kAccF32;

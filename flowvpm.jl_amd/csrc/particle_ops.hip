@@ -348,7 +348,7 @@ int launch_update_states(vpm_field f, double a, double b, double dt, const doubl
     hipLaunchKernelGGL(update_states_kernel, dim3(nb(f->np)), dim3(kBlock), 0, f->stream, f->P, f->np, a, b, dt,
                        Uinf[0], Uinf[1], Uinf[2], fr, gr, zeta0, transposed);
     VPM_CHECK_LAUNCH("update_particle_states");
-    f->perm_valid = false;
+    f->moved();
     return VPM_OK;
 }
 

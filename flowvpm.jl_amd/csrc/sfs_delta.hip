@@ -477,7 +477,7 @@ __global__ __launch_bounds__(kBlock) void sfsd_store_kernel(const double* __rest
     M[5] = rec[RSFS + 2] + de[2 * ld + k];
 }
 
-int launch_sfs_delta(vpm_field f, int kernel, int transposed, double alpha)
+int launch_sfs_delta(vpm_field f, int kernel, int transposed, double alpha, Order order)
 {
     const int64_t np = f->np;
     if (np == 0) return VPM_OK;
@@ -485,7 +485,7 @@ int launch_sfs_delta(vpm_field f, int kernel, int transposed, double alpha)
     const int64_t ld = np;
     int rc;
     const uint32_t* perm = nullptr;
-    if (np > 1 && (rc = sort_field(f, perm))) return rc;
+    if ((rc = sort_field(f, order, perm))) return rc;
     // scratch: pos 3, J 9, dJ 9, dE 3 doubles; gs, gz float4; tile boxes; cut float
     const size_t nd = 24 * (size_t)np;
     const int64_t ntile = (np + kTile - 1) / kTile;

@@ -34,6 +34,15 @@
 //    tile), computed once, tell both kernels who takes which group.
 //  * The FP32 accumulators are added to FP64 sums after every tile; the
 //    polynomials in t are formed once per target in FP64.
+// Measured: U/J of the 2^20 jet 702 -> 345 ms (1.57e12 -> 3.2e12 pairs/s), of
+// the 65,536 cloud 3.84 -> 2.60 ms and of the leapfrog rings 3.41 -> 1.92 ms;
+// error against 64 bits of U unchanged (1.6e-7 on the cloud), of J 4.5e-7 ->
+// 3.0e-7 (rest kernel).  The far kernel is bound by the VALU: per pair one
+// rsq (8.3 cycles per wave), three products (2.6 each), two packed conversions
+// of two (4.6) and a fma_mix (4.4) are 25-32 cycles per 64 pairs; the matrix
+// products (7 per 1,024 pairs, 15 cycles per 64) run beside them (two of the
+// three left out changes nothing).  It runs at 44: the clock falls from 2.35
+// to 1.93 GHz under both, and staging and folding add 11 %.
 #include <algorithm>
 #include <cfloat>
 
@@ -51,9 +60,19 @@ constexpr int kColLd = kTile + 8;    // halves per column row in LDS: 33 x 16 by
 constexpr int kColShift = 13;        // columns are scaled by 2^13
 constexpr float kLowScale = 64.f;    // scale of the low FP16 part of a position
 constexpr float kSqScale = 4096.f;   // scale of s^2 and t^2 in the r^2 product
-constexpr int64_t kFarMin = 2048;    // fewest targets and sources
-constexpr int64_t kFarBlocks = 2048; // blocks of a launch, far kernel
-constexpr int64_t kRestBlocks = 4096; // and rest kernel
+// The far kernel pays from about 16,384 particles (U/J of the cloud, the jet
+// and the leapfrog rings, with and without it: 0.279 / 0.287, 0.255 / 0.264 and
+// 0.271 / 0.313 ms at 16,384; 0.139 / 0.110 ms for the cloud at 8,192, where
+// boxes of 64 particles are too large for most of their pairs to be far).
+constexpr int64_t kFarPairs = (int64_t)1 << 28;
+constexpr int64_t kFarMin = 2048;
+// Blocks of a launch.  The far kernel's blocks do equal work per tile; 2,048
+// or 8,192 of them measure the same at N = 65,536, and fewer splits leave
+// fewer partial sums.  The rest kernel's work per wave is uneven (a wave whose
+// targets are scattered reaches most sources), so it has at least 16 splits:
+// 352 ms at 2^20 with 16 or more, 358 with 8, 401 with 2.
+constexpr int64_t kFarBlocks = 2048;
+constexpr int64_t kRestBlocks = 4096;
 constexpr int64_t kRestMin = 16;
 constexpr int kFarThreads = 512;     // threads of a block of 256 targets
 
@@ -501,7 +520,7 @@ __global__ __launch_bounds__(kBlock, 4) void uj_rest_kernel(
 bool far_applies(int kernel, int precision, int64_t nt, int64_t ns)
 {
     const bool cheap = kernel == VPM_KERNEL_GAUSSIANERF || kernel == VPM_KERNEL_GAUSSIAN;
-    return cheap && precision == VPM_PREC_F32C && nt >= kFarMin && ns >= kFarMin;
+    return cheap && precision == VPM_PREC_F32C && nt >= kFarMin && ns >= kFarMin && nt * ns >= kFarPairs;
 }
 
 static int64_t up256(int64_t b) { return (b + 255) & ~(int64_t)255; }

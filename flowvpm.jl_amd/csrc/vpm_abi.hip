@@ -12,7 +12,7 @@
 #include <string>
 #include <vector>
 
-#include "vpm_internal.h"
+#include "uj_far.h"
 
 namespace vpm {
 
@@ -131,7 +131,7 @@ static int sync(vpm_field f)
 }
 
 // UJ_direct body on a locked field (src/FLOWVPM_UJ.jl:21-37)
-static int uj_direct_locked(vpm_field f, const vpm_config* cfg, uint32_t flags)
+static int uj_direct_locked(vpm_field f, const vpm_config* cfg, uint32_t flags, bool step = false)
 {
     int rc;
     const bool far64 = flags & VPM_UJ_F64_FAR;
@@ -141,13 +141,21 @@ static int uj_direct_locked(vpm_field f, const vpm_config* cfg, uint32_t flags)
     if (flags & VPM_UJ_RESET_SFS) if ((rc = launch_reset(f, 1))) return rc;
     const int prec = far64 ? kPrecF64Far : cfg->precision;
     const bool sort = (cfg->precision == VPM_PREC_F32C || far64) && !(flags & VPM_UJ_NO_SORT);
+    // The far kernel, where the spatial order makes groups far.  E_str on
+    // smooth fields is a difference of nearly equal J (1e-3 of it is the FP32
+    // rounding of J on thin rings), so a call that returns E_str keeps the
+    // rounding of the VALU kernel; the steps of small fields too.
+    const bool far = sort && far_applies(cfg->kernel, prec, f->np, f->np) &&
+                     (step ? f->np >= kFarStepMin : !(flags & VPM_UJ_SFS));
+    const Order order = !sort ? kStorage : far ? kHilbert : kZOrder;
     Staged st;
-    if ((rc = stage_field(f, cfg->kernel, prec, sort, st))) return rc;
-    if ((rc = launch_uj(f, st, 0, f->np, st, 0, f->np, cfg->kernel, prec))) return rc;
+    if ((rc = stage_field(f, cfg->kernel, prec, order, st))) return rc;
+    if ((rc = launch_uj(f, st, 0, f->np, st, 0, f->np, cfg->kernel, prec, far))) return rc;
     if (flags & VPM_UJ_SFS) {
         if (far64) return launch_estr_f64far(f, cfg->kernel, cfg->transposed);
         const uint32_t* perm = nullptr;
-        if (cfg->precision == VPM_PREC_F32C && (rc = sort_field(f, perm))) return rc;
+        // NO_SORT orders U/J only
+        if (cfg->precision == VPM_PREC_F32C && (rc = sort_field(f, far ? kHilbert : kZOrder, perm))) return rc;
         if ((rc = launch_estr_impl(f, cfg->kernel, cfg->transposed, cfg->precision, perm))) return rc;
     }
     return VPM_OK;
@@ -155,13 +163,13 @@ static int uj_direct_locked(vpm_field f, const vpm_config* cfg, uint32_t flags)
 
 // uj_flags: VPM_UJ_F64_FAR or 0, as the step's own U/J evaluations
 static int sfs_before_locked(vpm_field f, const vpm_config* cfg, double alpha, double minC, double maxC,
-                             uint32_t uj_flags = 0)
+                             uint32_t uj_flags = 0, bool step = false)
 {
     if (minC < 0 || maxC < 0 || minC > maxC)                         // subfilterscale.jl:455-461
         return fail(VPM_EINVAL, "Invalid C bounds");
     int rc;
     if ((rc = launch_scale_sigma(f, alpha, 0))) return rc;
-    if ((rc = uj_direct_locked(f, cfg, VPM_UJ_RESET | VPM_UJ_RESET_SFS | VPM_UJ_SFS | uj_flags))) return rc;
+    if ((rc = uj_direct_locked(f, cfg, VPM_UJ_RESET | VPM_UJ_RESET_SFS | VPM_UJ_SFS | uj_flags, step))) return rc;
     if ((rc = launch_sfs_store_test(f, cfg->transposed))) return rc;
     return launch_scale_sigma(f, alpha, 1);
 }
@@ -255,7 +263,7 @@ int vpm_destroy(vpm_field f)
         std::lock_guard<std::mutex> lock(f->mu);
         (void)hipSetDevice(f->device);
         (void)hipStreamSynchronize(f->stream);
-        DevBuf* bufs[] = {&f->pos, &f->gs, &f->cut, &f->g64, &f->part, &f->keys, &f->keys2, &f->perm,
+        DevBuf* bufs[] = {&f->pos, &f->gs, &f->cut, &f->g64, &f->part, &f->far, &f->keys, &f->keys2, &f->perm[0], &f->perm[1],
                           &f->iota, &f->sorttmp, &f->bbox, &f->flag, &f->adj, &f->rng, &f->bar, &f->xfer,
                           &f->lrec};
         for (DevBuf* b : bufs) release(*b);
@@ -302,7 +310,7 @@ int vpm_set_particles(vpm_field f, const double* particles, int64_t np)
         if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync(H2D)");
     }
     f->np = np;
-    f->perm_valid = false;
+    f->moved();
     return sync(f);
 }
 
@@ -325,7 +333,7 @@ int vpm_add_particles(vpm_field f, const double* particles, int64_t n)
                                   hipMemcpyHostToDevice, f->stream);
     if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync(H2D)");
     f->np += n;
-    f->perm_valid = false;
+    f->moved();
     return sync(f);
 }
 
@@ -347,7 +355,7 @@ int vpm_remove_particle(vpm_field f, int64_t i)
     e = hipMemsetAsync(f->P + last * NF + RU, 0, sizeof(double) * (RM - RU), f->stream);
     if (e != hipSuccess) return hip_fail(e, "hipMemsetAsync");
     f->np = last;
-    f->perm_valid = false;
+    f->moved();
     return sync(f);
 }
 
@@ -413,9 +421,11 @@ int vpm_uj_direct_fields(vpm_field target, vpm_field source, const vpm_config* c
         std::lock_guard<std::mutex> lock(target->mu);
         if (int rc = set_device(target)) return rc;
         Staged st;
-        const bool sort = cfg->precision == VPM_PREC_F32C;
-        if (int rc = stage_field(target, cfg->kernel, cfg->precision, sort, st)) return rc;
-        if (int rc = launch_uj(target, st, 0, target->np, st, 0, target->np, cfg->kernel, cfg->precision)) return rc;
+        const bool far = far_applies(cfg->kernel, cfg->precision, target->np, target->np);
+        const Order order = cfg->precision != VPM_PREC_F32C ? kStorage : far ? kHilbert : kZOrder;
+        if (int rc = stage_field(target, cfg->kernel, cfg->precision, order, st)) return rc;
+        if (int rc = launch_uj(target, st, 0, target->np, st, 0, target->np, cfg->kernel, cfg->precision, far))
+            return rc;
         return sync(target);
     }
     if (target->device != source->device) return fail(VPM_EINVAL, "fields live on different devices");
@@ -423,12 +433,14 @@ int vpm_uj_direct_fields(vpm_field target, vpm_field source, const vpm_config* c
     vpm_field a = target < source ? target : source, b = target < source ? source : target;
     std::lock_guard<std::mutex> la(a->mu), lb(b->mu);
     if (int rc = set_device(target)) return rc;
-    const bool sort = cfg->precision == VPM_PREC_F32C;
+    const bool far = far_applies(cfg->kernel, cfg->precision, target->np, source->np);
+    const Order order = cfg->precision != VPM_PREC_F32C ? kStorage : far ? kHilbert : kZOrder;
     Staged ss, ts;
-    if (int rc = stage_field(source, cfg->kernel, cfg->precision, sort, ss)) return rc;
+    if (int rc = stage_field(source, cfg->kernel, cfg->precision, order, ss)) return rc;
     if (int rc = sync(source)) return rc;          // source staging is on the source stream
-    if (int rc = stage_field(target, cfg->kernel, cfg->precision, sort, ts)) return rc;
-    if (int rc = launch_uj(target, ts, 0, target->np, ss, 0, source->np, cfg->kernel, cfg->precision)) return rc;
+    if (int rc = stage_field(target, cfg->kernel, cfg->precision, order, ts)) return rc;
+    if (int rc = launch_uj(target, ts, 0, target->np, ss, 0, source->np, cfg->kernel, cfg->precision, far))
+        return rc;
     return sync(target);
 }
 
@@ -572,7 +584,7 @@ int vpm_estr_direct(vpm_field f, const vpm_config* cfg)
     if (int rc = check_cfg(cfg)) return rc;
     const uint32_t* perm = nullptr;
     if (cfg->precision == VPM_PREC_F32C)
-        if (int rc = sort_field(f, perm)) return rc;
+        if (int rc = sort_field(f, kZOrder, perm)) return rc;
     if (int rc = launch_estr_impl(f, cfg->kernel, cfg->transposed, cfg->precision, perm)) return rc;
     return sync(f);
 }
@@ -645,6 +657,8 @@ static int rk3_step_locked(vpm_field f, vpm_step_config* s, double dt, int32_t r
         return fail(VPM_EINVAL, "CoreSpreading requires the Gaussian-erf kernel");
     const double zeta0 = zeta0_of(cfg->kernel);                    // timeintegration.jl:398
     const bool sfs = s->sfs != 0;
+    // the spatial order of the step's U/J evaluations (uj_direct_locked)
+    const Order order = far_applies(cfg->kernel, cfg->precision, f->np, f->np) && f->np >= kFarStepMin ? kHilbert : kZOrder;
     int rc;
     bool reset_needed = false, unconverged = false;
     const size_t rec = sizeof(double) * NF * (size_t)f->np;
@@ -666,10 +680,11 @@ static int rk3_step_locked(vpm_field f, vpm_step_config* s, double dt, int32_t r
                               cfg->kernel != VPM_KERNEL_SINGULAR && 1.0 - s->sfs_alpha <= 0.01 &&
                               s->sfs_alpha < 1.0;
         if (sfs && first && !sfs_diff)
-            if ((rc = sfs_before_locked(f, cfg, s->sfs_alpha, s->sfs_minC, s->sfs_maxC, (uint32_t)s->uj_flags)))
+            if ((rc = sfs_before_locked(f, cfg, s->sfs_alpha, s->sfs_minC, s->sfs_maxC, (uint32_t)s->uj_flags,
+                                        true)))
                 return rc;
         const uint32_t fl = VPM_UJ_RESET | (sfs ? (VPM_UJ_RESET_SFS | VPM_UJ_SFS) : 0u) | (uint32_t)s->uj_flags;
-        if ((rc = uj_direct_locked(f, cfg, fl))) return rc;        // :422
+        if ((rc = uj_direct_locked(f, cfg, fl, true))) return rc;  // :422
         if (tape && f->np > 0) {
             hipError_t e = hipMemcpyAsync((char*)tape->rec.p + st * rec, f->P, rec, hipMemcpyDeviceToDevice,
                                           f->stream);
@@ -678,7 +693,7 @@ static int rk3_step_locked(vpm_field f, vpm_step_config* s, double dt, int32_t r
         if (sfs_diff) {
             if (s->sfs_minC < 0 || s->sfs_maxC < 0 || s->sfs_minC > s->sfs_maxC)   // subfilterscale.jl:455-461
                 return fail(VPM_EINVAL, "Invalid C bounds");
-            if ((rc = launch_sfs_delta(f, cfg->kernel, cfg->transposed, s->sfs_alpha))) return rc;
+            if ((rc = launch_sfs_delta(f, cfg->kernel, cfg->transposed, s->sfs_alpha, order))) return rc;
         }
         if (sfs && first)
             if ((rc = sfs_after_locked(f, cfg, s->sfs_alpha, s->sfs_rlxf, s->sfs_minC, s->sfs_maxC,
@@ -708,7 +723,7 @@ static int rk3_step_locked(vpm_field f, vpm_step_config* s, double dt, int32_t r
     }
     if (relax_now && s->relax) {                                    // :437-458
         if ((rc = launch_reset(f, 0))) return rc;
-        if ((rc = uj_direct_locked(f, cfg, VPM_UJ_RESET | (uint32_t)s->uj_flags))) return rc;
+        if ((rc = uj_direct_locked(f, cfg, VPM_UJ_RESET | (uint32_t)s->uj_flags, true))) return rc;
         if ((rc = launch_relax(f, s->rlxf, s->relax == 2))) return rc;
     }
     if ((rc = launch_update_uprev(f))) return rc;                   // particlefield.jl:443-455
@@ -842,7 +857,7 @@ int vpm_rk3_step_adjoint(vpm_tape t, double* bar)
     for (int st = 2; st >= 0; --st) {
         e = hipMemcpyAsync(f->P, (const char*)t->rec.p + st * rec, rec, hipMemcpyDeviceToDevice, f->stream);
         if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync(restore stage)");
-        f->perm_valid = false;
+        f->moved();
         if ((rc = launch_update_states_adjoint(f, B, coef[st][0], coef[st][1], t->dt, s.f, s.g, s.uj.transposed,
                                                ab.U, ab.J)))
             return rc;

@@ -76,8 +76,10 @@ struct vpm_field_s {
     vpm::DevBuf cut;                 // float  [cap]     far-field r^2 threshold
     vpm::DevBuf g64;                 // double4 [cap]    (Gamma, sigma)
     vpm::DevBuf part;                // double partial sums [K][acc][ld]
-    vpm::DevBuf keys, keys2, perm, iota, sorttmp;
-    bool perm_valid = false;         // perm matches the current positions
+    vpm::DevBuf far;                 // boxes and words of the far kernel (uj_far.h)
+    vpm::DevBuf keys, keys2, perm[2], iota, sorttmp;
+    bool perm_valid[2] = {};         // perm[Z order, Hilbert order] matches the current positions
+    void moved() { perm_valid[0] = perm_valid[1] = false; }   // positions or np changed
     vpm::DevBuf bbox;                // double [6 + partials]
     vpm::DevBuf flag;                // int device error flag
     vpm::DevBuf adj;                 // adjoint / E_str staging scratch
@@ -146,15 +148,19 @@ struct Staged {
     const uint32_t* perm;  // sorted index -> particle index, or nullptr
 };
 
+// Order of the staged particles: storage order, or sorted along a curve.
+enum Order : int { kStorage = 0, kZOrder = 1, kHilbert = 2 };
+
 // With an Arena, the scratch of these calls (sort keys and permutation,
 // staged sources, partial sums) is taken from it instead of the field's
 // grow-only buffers, nothing is allocated, and the permutation is not kept
-// for later calls.  launch_uj's kmax > 0 caps the number of source splits.
-int sort_field(vpm_field f, const uint32_t*& perm, Arena* ar = nullptr);
-int stage_field(vpm_field f, int kernel, int precision, bool sort, Staged& out, Arena* ar = nullptr);
+// for later calls.  launch_uj's kmax > 0 caps the number of source splits;
+// far (where far_applies) takes the far field to the matrix cores.
+int sort_field(vpm_field f, Order order, const uint32_t*& perm, Arena* ar = nullptr);
+int stage_field(vpm_field f, int kernel, int precision, Order order, Staged& out, Arena* ar = nullptr);
 int launch_uj(vpm_field ft, const Staged& T, int64_t t0, int64_t nt,
               const Staged& S, int64_t s0, int64_t s1, int kernel, int precision,
-              Arena* ar = nullptr, int64_t kmax = 0);
+              bool far, Arena* ar = nullptr, int64_t kmax = 0);
 // Source splits of an all-pairs launch over nt targets and ns sources (at
 // most kmax when kmax > 0): K chunks of `chunk` sources, a multiple of the tile.
 void choose_split(int64_t nt, int64_t ns, int64_t kmax, int64_t& K, int64_t& chunk);
@@ -202,7 +208,7 @@ int launch_core_spreading_reset(vpm_field f, int kernel, int precision, double s
                                 int iterror, int* iters, double res[3]);
 int launch_rbf_cg(vpm_field f, int kernel, int precision, int itmax, double tol, int iterror, int* iters,
                   double res[3]);
-int launch_sfs_delta(vpm_field f, int kernel, int transposed, double alpha);
+int launch_sfs_delta(vpm_field f, int kernel, int transposed, double alpha, Order order);
 int launch_gather_rows(vpm_field f, int row0, int nrows, double* out);
 int launch_zeta_ranges(vpm_field f, int kernel, int precision, const int64_t* tb, const int64_t* te,
                        const int64_t* sb, const int64_t* se, int64_t npairs);

@@ -265,7 +265,7 @@ int launch_zeta(vpm_field f, int kernel, int precision)
         if ((e = hipGetLastError()) != hipSuccess) return hip_fail(e, "zeta_f64");
         timing_end(f, 4);
     } else {
-        if (np > 1 && (rc = sort_field(f, perm))) return rc;
+        if ((rc = sort_field(f, kZOrder, perm))) return rc;
         if ((rc = ensure(f->pos, sizeof(double) * 3 * (size_t)ld))) return rc;
         const int64_t ntile = (np + kTile - 1) / kTile;
         if ((rc = ensure(f->adj, (sizeof(float4) + sizeof(float2)) * (size_t)np + 64 * (size_t)ntile + 16)))
