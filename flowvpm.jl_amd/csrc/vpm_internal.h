@@ -80,7 +80,7 @@ struct vpm_field_s {
     vpm::DevBuf keys, keys2, perm[2], iota, sorttmp;
     bool perm_valid[2] = {};         // perm[Z order, Hilbert order] matches the current positions
     void moved() { perm_valid[0] = perm_valid[1] = false; }   // positions or np changed
-    vpm::DevBuf bbox;                // double [6 + partials]
+    vpm::DevBuf bbox;                // double [6][blocks] partial boxes
     vpm::DevBuf flag;                // int device error flag
     vpm::DevBuf adj;                 // adjoint / E_str staging scratch
     vpm::DevBuf rng;                 // leaf-pair range lists
