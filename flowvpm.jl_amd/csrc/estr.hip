@@ -224,15 +224,12 @@ __global__ __launch_bounds__(kBlock) void estr_finalize_kernel(const double* __r
                                                               const uint32_t* __restrict__ perm, int transposed,
                                                               double* __restrict__ P)
 {
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i >= np) return;
+    int64_t i;
+    double a[6];
+    if (!sum_splits(part, pld, K, np, i, a)) return;
     const int64_t p = perm ? (int64_t)perm[i] : i;
     double* rec = P + p * NF;
     if (rec[RSTATIC] != 0) return;                      // subfilterscale_models.jl:63
-    double a[6] = {0, 0, 0, 0, 0, 0};
-    for (int k = 0; k < K; ++k)
-#pragma unroll
-        for (int c = 0; c < 6; ++c) a[c] += part[((int64_t)k * 6 + c) * pld + i];
     const int64_t ib = (i / kBlock) * kBlock;
     double Jp[9];
 #pragma unroll
@@ -539,7 +536,7 @@ int launch_estr_impl(vpm_field f, int kernel, int transposed, int precision, con
     e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "estr_f32c");
     timing_end(f, 2);
-    hipLaunchKernelGGL(estr_finalize_kernel, dim3(nblk(np)), dim3(kBlock), 0, f->stream, part, np, (int)K, J, ld, np,
+    hipLaunchKernelGGL(estr_finalize_kernel, dim3(sum_blocks(np)), dim3(kBlock), 0, f->stream, part, np, (int)K, J, ld, np,
                        perm, transposed, f->P);
     e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "estr_finalize");

@@ -203,22 +203,15 @@ __global__ __launch_bounds__(kBlock, 5) void uj_f64far_kernel(
 }
 
 // ------------------------------------------------------------- finalize
-// Sums the K partials of each target in split order and adds the total onto
+// Sums the K partials of each target in a fixed order and adds the total onto
 // U and J of the particle record (buffer_to_target_system!, fmm.jl:170-176).
 __global__ __launch_bounds__(kBlock) void finalize_f32c_kernel(
     const double* __restrict__ part, int64_t pld, int K, int64_t nt,
     const uint32_t* __restrict__ perm, int64_t t0, double* __restrict__ P)
 {
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i >= nt) return;
+    int64_t i;
     double a[kAccF32];
-#pragma unroll
-    for (int c = 0; c < kAccF32; ++c) a[c] = 0.0;
-    for (int k = 0; k < K; ++k) {
-        const double* p = part + (int64_t)k * kAccF32 * pld + i;
-#pragma unroll
-        for (int c = 0; c < kAccF32; ++c) a[c] += p[c * pld];
-    }
+    if (!sum_splits(part, pld, K, nt, i, a)) return;
     const int64_t idx = perm ? (int64_t)perm[t0 + i] : t0 + i;
     add_f32c_to_record(P + idx * NF, a);
 }
@@ -227,16 +220,9 @@ __global__ __launch_bounds__(kBlock) void finalize_f64_kernel(
     const double* __restrict__ part, int64_t pld, int K, int64_t nt,
     const uint32_t* __restrict__ perm, int64_t t0, double* __restrict__ P)
 {
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i >= nt) return;
+    int64_t i;
     double a[kAccF64];
-#pragma unroll
-    for (int c = 0; c < kAccF64; ++c) a[c] = 0.0;
-    for (int k = 0; k < K; ++k) {
-        const double* p = part + (int64_t)k * kAccF64 * pld + i;
-#pragma unroll
-        for (int c = 0; c < kAccF64; ++c) a[c] += p[c * pld];
-    }
+    if (!sum_splits(part, pld, K, nt, i, a)) return;
     const int64_t idx = perm ? (int64_t)perm[t0 + i] : t0 + i;
     double* rec = P + idx * NF;
 #pragma unroll
@@ -648,7 +634,7 @@ static int launch_uj_split(vpm_field ft, const Staged& T, int64_t nt, const Stag
         timing_begin(ft);
         if ((rc = launch_uj_far(ft->stream, T, t0, n, S, ns, kernel, k, fp, part))) return rc;
         timing_end(ft, 0);
-        hipLaunchKernelGGL(finalize_f32c_kernel, dim3(nblocks(n)), dim3(kBlock), 0, ft->stream, (const double*)part,
+        hipLaunchKernelGGL(finalize_f32c_kernel, dim3(sum_blocks(n)), dim3(kBlock), 0, ft->stream, (const double*)part,
                            n, (int)(k.far + k.rest), n, T.perm, t0, ft->P);
         VPM_LAUNCH_CHECK("finalize_f32c");
     }
@@ -689,7 +675,7 @@ int launch_uj(vpm_field ft, const Staged& T, int64_t t0, int64_t nt, const Stage
         }
         VPM_LAUNCH_CHECK("uj_f64");
         timing_end(ft, 1);
-        hipLaunchKernelGGL(finalize_f64_kernel, dim3(nblocks(nt)), dim3(kBlock), 0, ft->stream, part, pld,
+        hipLaunchKernelGGL(finalize_f64_kernel, dim3(sum_blocks(nt)), dim3(kBlock), 0, ft->stream, part, pld,
                            (int)K, nt, T.perm, t0, ft->P);
         VPM_LAUNCH_CHECK("finalize_f64");
         return VPM_OK;
@@ -711,7 +697,7 @@ int launch_uj(vpm_field ft, const Staged& T, int64_t t0, int64_t nt, const Stage
         }
         VPM_LAUNCH_CHECK("uj_f64far");
         timing_end(ft, 1);
-        hipLaunchKernelGGL(finalize_f32c_kernel, dim3(nblocks(nt)), dim3(kBlock), 0, ft->stream, part, pld,
+        hipLaunchKernelGGL(finalize_f32c_kernel, dim3(sum_blocks(nt)), dim3(kBlock), 0, ft->stream, part, pld,
                            (int)K, nt, T.perm, t0, ft->P);
         VPM_LAUNCH_CHECK("finalize_f32c");
         return VPM_OK;
@@ -732,7 +718,7 @@ int launch_uj(vpm_field ft, const Staged& T, int64_t t0, int64_t nt, const Stage
     }
     VPM_LAUNCH_CHECK("uj_f32c");
     timing_end(ft, 0);
-    hipLaunchKernelGGL(finalize_f32c_kernel, dim3(nblocks(nt)), dim3(kBlock), 0, ft->stream, part, pld,
+    hipLaunchKernelGGL(finalize_f32c_kernel, dim3(sum_blocks(nt)), dim3(kBlock), 0, ft->stream, part, pld,
                        (int)K, nt, T.perm, t0, ft->P);
     VPM_LAUNCH_CHECK("finalize_f32c");
     return VPM_OK;

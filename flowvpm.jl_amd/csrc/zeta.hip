@@ -213,13 +213,9 @@ __global__ __launch_bounds__(kBlock) void zeta_finalize_kernel(const double* __r
                                                                int64_t np, const uint32_t* __restrict__ perm,
                                                                double* __restrict__ P)
 {
-    const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (k >= np) return;
-    double a[3] = {0.0, 0.0, 0.0};
-    for (int s = 0; s < K; ++s) {
-        const double* p = part + (int64_t)s * 3 * pld + k;
-        for (int c = 0; c < 3; ++c) a[c] += p[c * pld];
-    }
+    int64_t k;
+    double a[3];
+    if (!sum_splits(part, pld, K, np, k, a)) return;
     const int64_t idx = perm ? (int64_t)perm[k] : k;
     double* rec = P + idx * NF;
     for (int c = 0; c < 3; ++c) rec[RJ + c] = a[c];
@@ -293,7 +289,7 @@ int launch_zeta(vpm_field f, int kernel, int precision)
         if ((e = hipGetLastError()) != hipSuccess) return hip_fail(e, "zeta_f32c");
         timing_end(f, 4);
     }
-    hipLaunchKernelGGL(zeta_finalize_kernel, dim3(nbt), dim3(kBlock), 0, f->stream, part, np, (int)K, np, perm,
+    hipLaunchKernelGGL(zeta_finalize_kernel, dim3(sum_blocks(np)), dim3(kBlock), 0, f->stream, part, np, (int)K, np, perm,
                        f->P);
     if ((e = hipGetLastError()) != hipSuccess) return hip_fail(e, "zeta_finalize");
     return VPM_OK;
