@@ -146,39 +146,62 @@ __device__ __forceinline__ void accum_pair(float dx, float dy, float dz, float F
     acc[13] = fmaf(hy, dz, acc[13]);   // Jhv[1][2]
 }
 
-// Far form of one pair: F' = r^-3, H'' = r^-5 (kernels with Far<K>::cheap),
-// or the full formula without the hi/lo correction (Winckelmans).
+// Separation and coefficients of one pair.
+struct PairCoef { float dx, dy, dz, Fp, Hpp; };
+
+// Far form: F' = r^-3, H'' = r^-5 (kernels with Far<K>::cheap), or the full
+// formula without the hi/lo correction (Winckelmans).
 template <int K>
-__device__ __forceinline__ void far_pair(float tx, float ty, float tz, const float4 a, const float4 b,
-                                         float (&acc)[kAccF32])
+__device__ __forceinline__ PairCoef far_coef(float tx, float ty, float tz, const float4 a, float sinv)
 {
-    const float dx = tx - a.x, dy = ty - a.y, dz = tz - a.z;
-    const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-    float Fp, Hpp;
+    PairCoef p;
+    p.dx = tx - a.x;
+    p.dy = ty - a.y;
+    p.dz = tz - a.z;
+    const float r2 = fmaf(p.dz, p.dz, fmaf(p.dy, p.dy, p.dx * p.dx));
     if constexpr (Far<K>::cheap) {
         const float ri = rsq(r2);
         const float ri2 = ri * ri;
-        Fp = ri2 * ri;
-        Hpp = Fp * ri2;
+        p.Fp = ri2 * ri;
+        p.Hpp = p.Fp * ri2;
     } else {
-        coef_full<K>(r2, b.w, Fp, Hpp);
+        coef_full<K>(r2, sinv, p.Fp, p.Hpp);
     }
-    accum_pair(dx, dy, dz, Fp, Hpp, b, acc);
+    return p;
 }
 
 // Near form: d from the hi/lo split (t - O = t'_hi + t'_lo to ~2^-48, so d
 // keeps FP32 relative accuracy however close the pair), full kernel formula.
 template <int K>
+__device__ __forceinline__ PairCoef near_coef(float tx, float ty, float tz, float tlx, float tly, float tlz,
+                                              const float4 a, float sinv, const float4 l)
+{
+    PairCoef p;
+    p.dx = (tx - a.x) + (tlx - l.x);
+    p.dy = (ty - a.y) + (tly - l.y);
+    p.dz = (tz - a.z) + (tlz - l.z);
+    const float r2 = fmaf(p.dz, p.dz, fmaf(p.dy, p.dy, p.dx * p.dx));
+    coef_full<K>(r2, sinv, p.Fp, p.Hpp);
+    return p;
+}
+
+__device__ __forceinline__ void accum_pair(const PairCoef& p, const float4 b, float (&acc)[kAccF32])
+{
+    accum_pair(p.dx, p.dy, p.dz, p.Fp, p.Hpp, b, acc);
+}
+
+template <int K>
+__device__ __forceinline__ void far_pair(float tx, float ty, float tz, const float4 a, const float4 b,
+                                         float (&acc)[kAccF32])
+{
+    accum_pair(far_coef<K>(tx, ty, tz, a, b.w), b, acc);
+}
+
+template <int K>
 __device__ __forceinline__ void near_pair(float tx, float ty, float tz, float tlx, float tly, float tlz,
                                           const float4 a, const float4 b, const float4 l, float (&acc)[kAccF32])
 {
-    const float dx = (tx - a.x) + (tlx - l.x);
-    const float dy = (ty - a.y) + (tly - l.y);
-    const float dz = (tz - a.z) + (tlz - l.z);
-    const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-    float Fp, Hpp;
-    coef_full<K>(r2, b.w, Fp, Hpp);
-    accum_pair(dx, dy, dz, Fp, Hpp, b, acc);
+    accum_pair(near_coef<K>(tx, ty, tz, tlx, tly, tlz, a, b.w, l), b, acc);
 }
 
 // Bounding box of the wave's targets (t'_hi), computed once per block; the
@@ -253,8 +276,13 @@ __device__ __forceinline__ void fold_u(float (&acc)[kAccF32], float (&sum)[kAccF
 // is near when its distance to the wave's target box is below q_far sigma
 // (then some lane may be near; the test is conservative).  The far and the
 // near sources are then visited by iterating over the set bits of the two
-// masks (scalar loop control), so the far loop body is straight-line.
-template <int K, int NG = kTile / 64, bool FOLD = (NG > 1)>
+// masks (scalar loop control), so the far loop body is straight-line.  TWO
+// takes two sources per iteration: their loads and coefficients overlap, and
+// the sums take them in order (the same results).  A kernel short of waves
+// gains (U/J of 3,001 / 8,000 particles 80 / 117 -> 73 / 111 us, Winckelmans
+// at 65,536 4.15 -> 4.02 ms); one that runs five waves per SIMD without it
+// loses more to the registers (rest kernel of the 65,536 cloud, +8 %).
+template <int K, int NG = kTile / 64, bool FOLD = (NG > 1), bool TWO = true>
 __device__ __forceinline__ void tile_f32c(int n, const float4* lpos, const float4* lgs, const float4* llo,
                                           float tx, float ty, float tz, float tlx, float tly, float tlz,
                                           const WaveBox& box, float (&acc)[kAccF32], float (&sum)[kAccF32],
@@ -287,6 +315,17 @@ __device__ __forceinline__ void tile_f32c(int n, const float4* lpos, const float
 #pragma unroll 16
             for (int s = 0; s < 64; ++s) far_pair<K>(tx, ty, tz, lpos[g * 64 + s], lgs[g * 64 + s], acc);
         } else {
+            while (TWO && (fb & (fb - 1))) {
+                const int s = g * 64 + __builtin_ctzll(fb);
+                fb &= fb - 1;
+                const int u = g * 64 + __builtin_ctzll(fb);
+                fb &= fb - 1;
+                const float4 bs = lgs[s], bu = lgs[u];
+                const PairCoef ps = far_coef<K>(tx, ty, tz, lpos[s], bs.w);
+                const PairCoef pu = far_coef<K>(tx, ty, tz, lpos[u], bu.w);
+                accum_pair(ps, bs, acc);
+                accum_pair(pu, bu, acc);
+            }
             while (fb) {
                 const int s = g * 64 + __builtin_ctzll(fb);
                 fb &= fb - 1;
@@ -300,19 +339,35 @@ __device__ __forceinline__ void tile_f32c(int n, const float4* lpos, const float
     // wave-uniform).  The wave-per-leaf list kernels (FOLD = false) fold
     // every 64 sources anyway.
     int nn = 0;
+    const auto fold = [&]() {
+        if constexpr (FOLD) {
+            if (++nn == kNearFold) {
+                fold_u(acc, sum, err);
+                nn = 0;
+            }
+        }
+    };
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
         uint64_t nb = near[g];
+        while (TWO && (nb & (nb - 1))) {
+            const int s = g * 64 + __builtin_ctzll(nb);
+            nb &= nb - 1;
+            const int u = g * 64 + __builtin_ctzll(nb);
+            nb &= nb - 1;
+            const float4 bs = lgs[s], bu = lgs[u];
+            const PairCoef ps = near_coef<K>(tx, ty, tz, tlx, tly, tlz, lpos[s], bs.w, llo[s]);
+            const PairCoef pu = near_coef<K>(tx, ty, tz, tlx, tly, tlz, lpos[u], bu.w, llo[u]);
+            accum_pair(ps, bs, acc);
+            fold();
+            accum_pair(pu, bu, acc);
+            fold();
+        }
         while (nb) {
             const int s = g * 64 + __builtin_ctzll(nb);
             nb &= nb - 1;
             near_pair<K>(tx, ty, tz, tlx, tly, tlz, lpos[s], lgs[s], llo[s], acc);
-            if constexpr (FOLD) {
-                if (++nn == kNearFold) {
-                    fold_u(acc, sum, err);
-                    nn = 0;
-                }
-            }
+            fold();
         }
     }
     (void)nn;

@@ -505,7 +505,7 @@ __global__ __launch_bounds__(kBlock, 4) void uj_rest_kernel(
                 float acc[kAccF32];
 #pragma unroll
                 for (int c = 0; c < kAccF32; ++c) acc[c] = 0.f;
-                tile_f32c<K, 1, true>(n, lpos, lgs, llo, tx, ty, tz, tlx, tly, tlz, box, acc, sum, err);
+                tile_f32c<K, 1, true, false>(n, lpos, lgs, llo, tx, ty, tz, tlx, tly, tlz, box, acc, sum, err);
                 fold_twosum(acc, sum, err);
             }
         }
