@@ -261,10 +261,12 @@ __device__ __forceinline__ double zeta_ref(double r)
     }
 }
 
-// One block per 256 targets (storage order); sources in storage order, whole
-// range per block (E_str is not the headline path; this is the oracle).
+// One block per 256 targets (storage order) and source split (whole tiles);
+// sources in storage order.  With every source in one block, the 64 blocks of
+// 16,384 particles left three quarters of the chip idle.
 template <int K>
-__global__ __launch_bounds__(kBlock) void estr_f64_kernel(double* __restrict__ P, int64_t np, int transposed)
+__global__ __launch_bounds__(kBlock) void estr_f64_kernel(const double* __restrict__ P, int64_t np, int transposed,
+                                                          int64_t chunk, double* __restrict__ part, int64_t pld)
 {
     __shared__ double lx[kTile][4];
     __shared__ double lg[kTile][4];
@@ -277,10 +279,10 @@ __global__ __launch_bounds__(kBlock) void estr_f64_kernel(double* __restrict__ P
     double JT[9];
 #pragma unroll
     for (int c = 0; c < 9; ++c) JT[c] = tr[RJ + c];
-    const bool tstatic = tr[RSTATIC] != 0;
     double s1 = 0, s2 = 0, s3 = 0;
-    for (int64_t base = 0; base < np; base += kTile) {
-        const int n = (int)min((int64_t)kTile, np - base);
+    const int64_t sb = (int64_t)blockIdx.y * chunk, se = min(sb + chunk, np);
+    for (int64_t base = sb; base < se; base += kTile) {
+        const int n = (int)min((int64_t)kTile, se - base);
         __syncthreads();
         if (tid < n) {
             const double* sr = P + (base + tid) * NF;
@@ -313,14 +315,27 @@ __global__ __launch_bounds__(kBlock) void estr_f64_kernel(double* __restrict__ P
             s3 += zeta_sgm * S3;
         }
     }
-    if (i < np && !tstatic) {
-        double* rec = P + i * NF;
-        rec[RSFS] += s1;
-        rec[RSFS + 1] += s2;
-        rec[RSFS + 2] += s3;
+    if (i < np) {
+        double* out = part + (int64_t)blockIdx.y * 3 * pld + i;
+        out[0] = s1;
+        out[pld] = s2;
+        out[2 * pld] = s3;
     }
 }
 #pragma clang fp contract(on)
+
+// SFS of the non-static particles += the sum of their split partials
+__global__ __launch_bounds__(kBlock) void estr_f64_finalize_kernel(const double* __restrict__ part, int64_t pld, int K,
+                                                                   int64_t np, double* __restrict__ P)
+{
+    int64_t i;
+    double a[3];
+    if (!sum_splits(part, pld, K, np, i, a)) return;
+    double* rec = P + i * NF;
+    if (rec[RSTATIC] != 0) return;                      // subfilterscale_models.jl:63
+#pragma unroll
+    for (int c = 0; c < 3; ++c) rec[RSFS + c] += a[c];
+}
 
 static inline unsigned nblk(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 
@@ -480,17 +495,33 @@ int launch_estr_impl(vpm_field f, int kernel, int transposed, int precision, con
     // The singular kernel's zeta is nonzero only at r = 0 (coincident pairs),
     // where the reference's (J_t - J_s) difference is exact: use FP64.
     if (precision == VPM_PREC_F64 || kernel == VPM_KERNEL_SINGULAR) {
+        // 4,096 blocks of equal work (16 waves per SIMD)
+        const int64_t tiles = (np + kTile - 1) / kTile;
+        int64_t K = std::min<int64_t>(std::max<int64_t>(1, 4096 / nblk(np)), tiles);
+        const int64_t chunk = ((tiles + K - 1) / K) * kTile;
+        K = (np + chunk - 1) / chunk;
+        if ((rc = ensure(f->part, sizeof(double) * 3 * (size_t)K * (size_t)np))) return rc;
+        double* part = (double*)f->part.p;
+        const dim3 grid(nblk(np), (unsigned)K);
         timing_begin(f);
         switch (kernel) {
-        case VPM_KERNEL_SINGULAR: hipLaunchKernelGGL(estr_f64_kernel<VPM_KERNEL_SINGULAR>, dim3(nblk(np)), dim3(kBlock), 0, f->stream, f->P, np, transposed); break;
-        case VPM_KERNEL_GAUSSIAN: hipLaunchKernelGGL(estr_f64_kernel<VPM_KERNEL_GAUSSIAN>, dim3(nblk(np)), dim3(kBlock), 0, f->stream, f->P, np, transposed); break;
-        case VPM_KERNEL_GAUSSIANERF: hipLaunchKernelGGL(estr_f64_kernel<VPM_KERNEL_GAUSSIANERF>, dim3(nblk(np)), dim3(kBlock), 0, f->stream, f->P, np, transposed); break;
-        case VPM_KERNEL_WINCKELMANS: hipLaunchKernelGGL(estr_f64_kernel<VPM_KERNEL_WINCKELMANS>, dim3(nblk(np)), dim3(kBlock), 0, f->stream, f->P, np, transposed); break;
+#define VPM_E64(KID)                                                                                              \
+    case KID:                                                                                                     \
+        hipLaunchKernelGGL(estr_f64_kernel<KID>, grid, dim3(kBlock), 0, f->stream, f->P, np, transposed, chunk,    \
+                           part, np);                                                                             \
+        break;
+            VPM_E64(VPM_KERNEL_SINGULAR) VPM_E64(VPM_KERNEL_GAUSSIAN) VPM_E64(VPM_KERNEL_GAUSSIANERF)
+            VPM_E64(VPM_KERNEL_WINCKELMANS)
+#undef VPM_E64
         default: return fail(VPM_EINVAL, "unknown kernel id");
         }
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return hip_fail(e, "estr_f64");
         timing_end(f, 2);
+        hipLaunchKernelGGL(estr_f64_finalize_kernel, dim3(sum_blocks(np)), dim3(kBlock), 0, f->stream,
+                           (const double*)part, np, (int)K, np, f->P);
+        e = hipGetLastError();
+        if (e != hipSuccess) return hip_fail(e, "estr_f64_finalize");
         return VPM_OK;
     }
     const int64_t ld = f->cap;
