@@ -449,12 +449,9 @@ def UJ_hip(pfield, *, reset=True, reset_sfs=False, sfs=False, kernel=None, preci
 
 
 def _copy_back(f, P, with_sfs):
-    tmp = np.empty_like(P)
-    f.get_particles(tmp, rows=(9, 27))
-    P[:, 9:27] = tmp[:, 9:27]
+    f.get_particles(P, rows=(9, 27))
     if with_sfs:
-        f.get_particles(tmp, rows=(39, 42))
-        P[:, 39:42] = tmp[:, 39:42]
+        f.get_particles(P, rows=(39, 42))
 
 
 def UJ_hip_fields(source, target, *, kernel=None, precision=None, device=None):
@@ -490,9 +487,7 @@ def p2p_ranges(pfield, tb, te, sb, se, *, kernel=None, precision=None, device=No
     cfg = make_config(kernel, precision, True)
     ptr = [a.ctypes.data_as(_lib._i64p) for a in arrs]
     check(lib().vpm_p2p_ranges(f.handle, C.byref(cfg), ptr[0], ptr[1], ptr[2], ptr[3], len(arrs[0])))
-    tmp = np.empty_like(P)
-    f.get_particles(tmp, rows=(9, 24))
-    P[:, 9:24] = tmp[:, 9:24]
+    f.get_particles(P, rows=(9, 24))
 
 
 def estr_ranges(pfield, tb, te, sb, se, *, kernel=None, precision=None, transposed=None, device=None):
@@ -512,9 +507,7 @@ def estr_ranges(pfield, tb, te, sb, se, *, kernel=None, precision=None, transpos
     cfg = make_config(kernel, precision, transposed)
     ptr = [a.ctypes.data_as(_lib._i64p) for a in arrs]
     check(lib().vpm_estr_ranges(f.handle, C.byref(cfg), ptr[0], ptr[1], ptr[2], ptr[3], len(arrs[0])))
-    tmp = np.empty_like(P)
-    f.get_particles(tmp, rows=(39, 42))
-    P[:, 39:42] = tmp[:, 39:42]
+    f.get_particles(P, rows=(39, 42))
 
 
 def zeta_ranges(pfield, tb, te, sb, se, *, kernel=None, precision=None, device=None):
@@ -533,9 +526,7 @@ def zeta_ranges(pfield, tb, te, sb, se, *, kernel=None, precision=None, device=N
     cfg = make_config(kernel, precision, True)
     ptr = [a.ctypes.data_as(_lib._i64p) for a in arrs]
     check(lib().vpm_zeta_ranges(f.handle, C.byref(cfg), ptr[0], ptr[1], ptr[2], ptr[3], len(arrs[0])))
-    tmp = np.empty_like(P)
-    f.get_particles(tmp, rows=(15, 18))
-    P[:, 15:18] = tmp[:, 15:18]
+    f.get_particles(P, rows=(15, 18))
 
 
 def Estr_hip(pfield, *, kernel=None, precision=None, transposed=None, device=None):
@@ -548,9 +539,7 @@ def Estr_hip(pfield, *, kernel=None, precision=None, transposed=None, device=Non
     f = _scratch_field(P.shape[0], 0 if device is None else device)
     f.set_particles(P)
     f.estr_direct(kernel, precision, transposed)
-    tmp = np.empty_like(P)
-    f.get_particles(tmp, rows=(39, 42))
-    P[:, 39:42] = tmp[:, 39:42]
+    f.get_particles(P, rows=(39, 42))
 
 
 # ---------------------------------------------------------------- time stepping

@@ -264,12 +264,14 @@ int vpm_destroy(vpm_field f)
         (void)hipSetDevice(f->device);
         (void)hipStreamSynchronize(f->stream);
         DevBuf* bufs[] = {&f->pos, &f->gs, &f->cut, &f->g64, &f->part, &f->far, &f->keys, &f->keys2, &f->perm[0], &f->perm[1],
-                          &f->iota, &f->sorttmp, &f->bbox, &f->flag, &f->adj, &f->rng, &f->bar, &f->xfer,
+                          &f->iota, &f->sorttmp, &f->bbox, &f->flag, &f->adj, &f->rng, &f->bar,
                           &f->lrec};
         for (DevBuf* b : bufs) release(*b);
-        if (f->hstage.p) (void)hipHostFree(f->hstage.p);
-        f->hstage.p = nullptr;
-        f->hstage.bytes = 0;
+        for (DevBuf* b : {&f->hstage, &f->ring}) {
+            if (b->p) (void)hipHostFree(b->p);
+            b->p = nullptr;
+            b->bytes = 0;
+        }
         for (vpm_tape t : f->tapes) {   // detach: the tape stays valid only for vpm_tape_destroy
             release(t->rec);
             t->f = nullptr;
@@ -297,21 +299,12 @@ int vpm_set_particles(vpm_field f, const double* particles, int64_t np)
     if (np < 0 || (np > 0 && !particles)) return fail(VPM_EINVAL, "bad particle array");
     if (np > f->cap) return fail(VPM_ERANGE, "PARTICLE OVERFLOW: " + std::to_string(np) + " > maxparticles " +
                                                   std::to_string(f->cap));
-    for (int64_t i = 0; i < np; ++i) {
-        const double* p = particles + i * NF;
-        for (int k = 0; k < 7; ++k)
-            if (!std::isfinite(p[k]))
-                return fail(VPM_EINVAL, "non-finite X/Gamma/sigma at particle " + std::to_string(i));
-        if (!(p[RSIG] > 0)) return fail(VPM_EINVAL, "sigma <= 0 at particle " + std::to_string(i));
-    }
-    if (np > 0) {
-        hipError_t e = hipMemcpyAsync(f->P, particles, sizeof(double) * NF * (size_t)np, hipMemcpyHostToDevice,
-                                      f->stream);
-        if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync(H2D)");
-    }
+    if (int rc = check_records(particles, np)) return rc;
+    if (np > 0)
+        if (int rc = upload_records(f, particles, 0, np)) return rc;
     f->np = np;
     f->moved();
-    return sync(f);
+    return np > 0 ? VPM_OK : sync(f);
 }
 
 int vpm_add_particles(vpm_field f, const double* particles, int64_t n)
@@ -321,20 +314,12 @@ int vpm_add_particles(vpm_field f, const double* particles, int64_t n)
     if (f->np + n > f->cap)
         return fail(VPM_ERANGE, "PARTICLE OVERFLOW. Max number of particles " + std::to_string(f->cap) +
                                     " has been reached");
-    for (int64_t i = 0; i < n; ++i) {
-        const double* p = particles + i * NF;
-        for (int k = 0; k < 7; ++k)
-            if (!std::isfinite(p[k]))
-                return fail(VPM_EINVAL, "non-finite X/Gamma/sigma at particle " + std::to_string(i));
-        if (!(p[RSIG] > 0)) return fail(VPM_EINVAL, "sigma <= 0 at particle " + std::to_string(i));
-    }
+    if (int rc = check_records(particles, n)) return rc;
     if (n == 0) return VPM_OK;
-    hipError_t e = hipMemcpyAsync(f->P + f->np * NF, particles, sizeof(double) * NF * (size_t)n,
-                                  hipMemcpyHostToDevice, f->stream);
-    if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync(H2D)");
+    if (int rc = upload_records(f, particles, f->np, n)) return rc;
     f->np += n;
     f->moved();
-    return sync(f);
+    return VPM_OK;
 }
 
 int vpm_remove_particle(vpm_field f, int64_t i)
@@ -366,30 +351,7 @@ int vpm_get_particles(vpm_field f, double* particles, int64_t np, int32_t row0, 
     if (row0 < 0 || row1 > NF || row0 >= row1) return fail(VPM_EINVAL, "bad row range");
     if (np == 0) return VPM_OK;
     if (!particles) return fail(VPM_EINVAL, "null output array");
-    hipError_t e;
-    if (row0 == 0 && row1 == NF) {   // whole records: one contiguous copy
-        e = hipMemcpyAsync(particles, f->P, sizeof(double) * NF * (size_t)np, hipMemcpyDeviceToHost, f->stream);
-        if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync(D2H)");
-        return sync(f);
-    }
-    // a row range: gather on the device, one contiguous copy, scatter on the
-    // host (a strided 2D copy of short rows is orders of magnitude slower)
-    const int nr = row1 - row0;
-    const size_t n = (size_t)np * (size_t)nr;
-    if (int rc = ensure(f->xfer, sizeof(double) * n)) return rc;
-    if (int rc = launch_gather_rows(f, row0, nr, (double*)f->xfer.p)) return rc;
-    std::vector<double> host;
-    try {
-        host.resize(n);
-    } catch (const std::exception&) {
-        return fail(VPM_ENOMEM, "host buffer of vpm_get_particles");
-    }
-    e = hipMemcpyAsync(host.data(), f->xfer.p, sizeof(double) * n, hipMemcpyDeviceToHost, f->stream);
-    if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync(D2H)");
-    if (int rc = sync(f)) return rc;
-    for (int64_t i = 0; i < np; ++i)
-        std::memcpy(particles + i * NF + row0, host.data() + (size_t)i * nr, sizeof(double) * nr);
-    return VPM_OK;
+    return download_rows(f, particles, np, row0, row1);
 }
 
 int vpm_get_np(vpm_field f, int64_t* np)

@@ -85,7 +85,7 @@ struct vpm_field_s {
     vpm::DevBuf adj;                 // adjoint / E_str staging scratch
     vpm::DevBuf rng;                 // leaf-pair range lists
     vpm::DevBuf bar;                 // cotangent records of the step adjoint
-    vpm::DevBuf xfer;                // gathered rows for partial downloads
+    vpm::DevBuf ring;                // pinned pieces of particle transfers (transfer.hip)
     vpm::DevBuf lrec;                // E_str / zeta list-kernel source records
     vpm::DevBuf hstage;              // pinned host staging of range plans (hipHostMalloc)
     bool profiling = false;
@@ -209,7 +209,13 @@ int launch_core_spreading_reset(vpm_field f, int kernel, int precision, double s
 int launch_rbf_cg(vpm_field f, int kernel, int precision, int itmax, double tol, int iterror, int* iters,
                   double res[3]);
 int launch_sfs_delta(vpm_field f, int kernel, int transposed, double alpha, Order order);
-int launch_gather_rows(vpm_field f, int row0, int nrows, double* out);
+// Particle transfers (transfer.hip).  check_records: VPM_EINVAL at the first
+// record with sigma <= 0 or a non-finite X, Gamma or sigma.  upload_records
+// fills records [first, first + np); download_rows writes rows [row0, row1) of
+// the first np records into a 46-stride array.  Both wait for the stream.
+int check_records(const double* p, int64_t np);
+int upload_records(vpm_field f, const double* src, int64_t first, int64_t np);
+int download_rows(vpm_field f, double* dst, int64_t np, int row0, int row1);
 int launch_zeta_ranges(vpm_field f, int kernel, int precision, const int64_t* tb, const int64_t* te,
                        const int64_t* sb, const int64_t* se, int64_t npairs);
 int launch_estr_ranges(vpm_field f, int kernel, int precision, int transposed, const int64_t* tb,
