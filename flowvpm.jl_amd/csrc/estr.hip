@@ -102,7 +102,7 @@ template <int K>
 __global__ __launch_bounds__(kBlock) void estr_f32c_kernel(
     const double* __restrict__ pos, const double* __restrict__ J, int64_t ld,
     const float4* __restrict__ gz, const float2* __restrict__ bc, const double* __restrict__ tbox, int64_t np,
-    int transposed, int64_t chunk, double* __restrict__ part, int64_t pld)
+    int transposed, double* __restrict__ part, int64_t pld)
 {
     __shared__ float4 lp[kTile];   // s'_hi x, y, z, a
     __shared__ float4 lg[kTile];   // Gamma x, y, z, b
@@ -126,20 +126,18 @@ __global__ __launch_bounds__(kBlock) void estr_f32c_kernel(
     block_box(wave_box(tx, ty, tz), wb, blo, bhi);
     const double org[3] = {ox, oy, oz};
 
-    const int64_t sb = (int64_t)blockIdx.y * chunk;
-    const int64_t se = min(sb + chunk, np);
     float sum[6], err[6];
 #pragma unroll
     for (int c = 0; c < 6; ++c) { sum[c] = 0.f; err[c] = 0.f; }
 
     __shared__ int nlist[kBlock];
     __shared__ int ncnt[kBlock / 64];
-    NearTiles near(tbox, sb / kTile, (se + kTile - 1) / kTile, org, blo, bhi, 1.0f, nlist, ncnt);
+    NearTiles near(tbox, blockIdx.y, (np + kTile - 1) / kTile, gridDim.y, org, blo, bhi, 1.0f, nlist, ncnt);
     for (int64_t tile; (tile = near.next()) >= 0;) {
         const int64_t base = tile * kTile;
         const int64_t j = base + tid;
         float4 p, g, q, l;
-        if (j < se) {
+        if (j < np) {
             const float4 gg = gz[j];
             const float2 b = bc[j];
             split_rel_e(pos[j], ox, p.x, l.x);
@@ -439,7 +437,7 @@ __global__ __launch_bounds__(kBlock) void estr_f64far_kernel(const double* __res
     block_box(wave_box((float)(tx - org[0]), (float)(ty - org[1]), (float)(tz - org[2])), wb, blo, bhi);
 
     double s1 = 0.0, s2 = 0.0, s3 = 0.0;
-    NearTiles near(tbox, 0, (np + kTile - 1) / kTile, org, blo, bhi, 1.0001f, nlist, ncnt);
+    NearTiles near(tbox, 0, (np + kTile - 1) / kTile, 1, org, blo, bhi, 1.0001f, nlist, ncnt);
     for (int64_t tile; (tile = near.next()) >= 0;) {
         const int64_t base = tile * kTile;
         const int64_t j = base + tid;
@@ -545,21 +543,19 @@ int launch_estr_impl(vpm_field f, int kernel, int transposed, int precision, con
                        (const float*)bc + 1, np, tbox);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "pack_estr");
-    // source splits, chunks of whole tiles: enough blocks to fill the chip,
-    // and up to 32 chunks of at least 16 tiles to spread the near-field work
-    // of blocks whose targets straddle a jump of the sort order (as for zeta)
+    // source splits (every K-th tile): enough blocks to fill the chip, and up
+    // to 32 to spread the near-field work of blocks whose targets straddle a
+    // jump of the sort order (as for zeta)
     const int64_t nb = (np + kBlock - 1) / kBlock;
     const int64_t tiles = (np + kTile - 1) / kTile;
     const int64_t k_fill = std::min<int64_t>((2560 + nb - 1) / nb, tiles);
     const int64_t k_spread = std::min<int64_t>(32, tiles / 16);
-    int64_t K = std::max<int64_t>(1, std::max(k_fill, k_spread));
-    const int64_t chunk = ((tiles + K - 1) / K) * kTile;
-    K = (np + chunk - 1) / chunk;
+    const int64_t K = std::max<int64_t>(1, std::max(k_fill, k_spread));
     if ((rc = ensure(f->part, sizeof(double) * 6 * (size_t)K * (size_t)np))) return rc;
     double* part = (double*)f->part.p;
     timing_begin(f);
     switch (kernel) {
-#define VPM_ES(KID) case KID: hipLaunchKernelGGL(estr_f32c_kernel<KID>, dim3(nblk(np), (unsigned)K), dim3(kBlock), 0, f->stream, pos, J, ld, gz, bc, (const double*)tbox, np, transposed, chunk, part, np); break;
+#define VPM_ES(KID) case KID: hipLaunchKernelGGL(estr_f32c_kernel<KID>, dim3(nblk(np), (unsigned)K), dim3(kBlock), 0, f->stream, pos, J, ld, gz, bc, (const double*)tbox, np, transposed, part, np); break;
         VPM_ES(VPM_KERNEL_GAUSSIAN) VPM_ES(VPM_KERNEL_GAUSSIANERF) VPM_ES(VPM_KERNEL_WINCKELMANS)
 #undef VPM_ES
     default: return fail(VPM_EINVAL, "unknown kernel id");

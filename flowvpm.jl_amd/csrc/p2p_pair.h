@@ -848,15 +848,18 @@ __device__ __forceinline__ float tile_gap2(const double* __restrict__ T, const d
     return g2;
 }
 
-// The near tiles of [t0, t1) for a block, in ascending order: kBlock tiles
-// are tested at once (one per thread, independent loads), the near ones are
+// The near tiles among t0, t0 + step, ... below t1 for a block, in ascending
+// order: kBlock tiles are tested at once (one per thread, independent loads), the near ones are
 // compacted into the __shared__ list, and next() walks the list.  A tile is
 // near when tile_gap2 < its largest cut times margin (the margin of the
 // kernel's per-source test).  All threads must call next() together: it
-// holds barriers and returns the same tile (or -1 at the end) to each.
+// holds barriers and returns the same tile (or -1 at the end) to each.  The
+// blocks of a target block's source splits take every step-th tile: its near
+// tiles are neighbours in the sort order, and contiguous splits left them to
+// one or two blocks (1.5 waves per SIMD at 65,536 particles).
 struct NearTiles {
     const double* tbox;
-    int64_t c0, t1;
+    int64_t c0, t1, step;
     const double* org;
     const float* blo;
     const float* bhi;
@@ -866,16 +869,16 @@ struct NearTiles {
     int cnt = 0, k = 0;
     int64_t cbase = 0;
 
-    __device__ NearTiles(const double* tb, int64_t first, int64_t end, const double (&o)[3], const float (&lo)[3],
+    __device__ NearTiles(const double* tb, int64_t first, int64_t end, int64_t st, const double (&o)[3], const float (&lo)[3],
                          const float (&hi)[3], float m, int* l, int* w)
-        : tbox(tb), c0(first), t1(end), org(o), blo(lo), bhi(hi), margin(m), list(l), wcnt(w) {}
+        : tbox(tb), c0(first), t1(end), step(st), org(o), blo(lo), bhi(hi), margin(m), list(l), wcnt(w) {}
 
     __device__ int64_t next()
     {
         while (k >= cnt) {
             if (c0 >= t1) return -1;
             const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-            const int64_t t = c0 + tid;
+            const int64_t t = c0 + tid * step;
             bool nr = false;
             if (t < t1) {
                 const double* T = tbox + 8 * t;
@@ -895,11 +898,11 @@ struct NearTiles {
             if (nr) list[off + __popcll(m & ((1ull << lane) - 1ull))] = tid;
             __syncthreads();
             cbase = c0;
-            c0 += kBlock;
+            c0 += kBlock * step;
             cnt = tot;
             k = 0;
         }
-        return cbase + list[k++];
+        return cbase + list[k++] * step;
     }
 };
 

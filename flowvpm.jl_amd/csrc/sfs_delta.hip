@@ -103,7 +103,7 @@ __global__ __launch_bounds__(kBlock) void dj_f32c_kernel(const double* __restric
                                                          const float4* __restrict__ sgs,
                                                          const float* __restrict__ scut,
                                                          const double* __restrict__ tbox, int64_t np, float delta,
-                                                         int64_t chunk, double* __restrict__ part)
+                                                         double* __restrict__ part)
 {
     __shared__ float4 lpos[kTile];
     __shared__ float4 lgs[kTile];
@@ -129,11 +129,10 @@ __global__ __launch_bounds__(kBlock) void dj_f32c_kernel(const double* __restric
     for (int c = 0; c < NA; ++c) { sum[c] = 0.f; err[c] = 0.f; }
     __shared__ int nlist[kBlock];
     __shared__ int ncnt[kBlock / 64];
-    const int64_t s0 = (int64_t)blockIdx.y * chunk, s1 = min(s0 + chunk, np);
-    NearTiles near(tbox, s0 / kTile, (s1 + kTile - 1) / kTile, org, blo, bhi, 1.0001f, nlist, ncnt);
+    NearTiles near(tbox, blockIdx.y, (np + kTile - 1) / kTile, gridDim.y, org, blo, bhi, 1.0001f, nlist, ncnt);
     for (int64_t tile; (tile = near.next()) >= 0;) {
         const int64_t base = tile * kTile;
-        const int n = (int)min((int64_t)kTile, s1 - base);
+        const int n = (int)min((int64_t)kTile, np - base);
         __syncthreads();
         if (tid < n) {
             const int64_t j = base + tid;
@@ -280,7 +279,7 @@ __global__ __launch_bounds__(kBlock) void de_f32c_kernel(const double* __restric
                                                          const double* __restrict__ dj, int64_t ld,
                                                          const float4* __restrict__ gz, const float* __restrict__ scut,
                                                          const double* __restrict__ tbox, int64_t np, float alpha,
-                                                         int transposed, int64_t chunk, double* __restrict__ part)
+                                                         int transposed, double* __restrict__ part)
 {
     __shared__ float4 lp[kTile];    // s'_hi, sigma (0: static)
     __shared__ float4 lg[kTile];    // Gamma, cut
@@ -309,11 +308,10 @@ __global__ __launch_bounds__(kBlock) void de_f32c_kernel(const double* __restric
     const float oma = 1.f - alpha;
     __shared__ int nlist[kBlock];
     __shared__ int ncnt[kBlock / 64];
-    const int64_t s0 = (int64_t)blockIdx.y * chunk, s1 = min(s0 + chunk, np);
-    NearTiles near(tbox, s0 / kTile, (s1 + kTile - 1) / kTile, org, blo, bhi, 1.0f, nlist, ncnt);
+    NearTiles near(tbox, blockIdx.y, (np + kTile - 1) / kTile, gridDim.y, org, blo, bhi, 1.0f, nlist, ncnt);
     for (int64_t tile; (tile = near.next()) >= 0;) {
         const int64_t base = tile * kTile;
-        const int n = (int)min((int64_t)kTile, s1 - base);
+        const int n = (int)min((int64_t)kTile, np - base);
         __syncthreads();
         if (tid < n) {
             const int64_t j = base + tid;
@@ -502,12 +500,10 @@ int launch_sfs_delta(vpm_field f, int kernel, int transposed, double alpha, Orde
     float* cut = (float*)(tbox + 8 * ntile);
     const unsigned nb = (unsigned)((np + kBlock - 1) / kBlock);
     const float delta = (float)(1.0 / alpha - 1.0);
-    // source chunks as for zeta and E_str (up to 32 of at least 16 tiles)
+    // source splits as for zeta and E_str
     const int64_t k_fill = std::min<int64_t>((2560 + nb - 1) / nb, ntile);
     const int64_t k_spread = std::min<int64_t>(32, ntile / 16);
-    int64_t nchunk = std::max<int64_t>(1, std::max(k_fill, k_spread));
-    const int64_t chunk = ((ntile + nchunk - 1) / nchunk) * kTile;
-    nchunk = (np + chunk - 1) / chunk;
+    const int64_t nchunk = std::max<int64_t>(1, std::max(k_fill, k_spread));
     if ((rc = ensure(f->part, sizeof(double) * 12 * (size_t)nchunk * (size_t)np))) return rc;
     double* part = (double*)f->part.p;
     const dim3 grid(nb, (unsigned)nchunk);
@@ -519,12 +515,12 @@ int launch_sfs_delta(vpm_field f, int kernel, int transposed, double alpha, Orde
         hipLaunchKernelGGL(tile_box_kernel<1>, dim3((unsigned)ntile), dim3(kBlock), 0, f->stream,                \
                            (const double*)pos, ld, (const float*)cut, np, tbox);                               \
         hipLaunchKernelGGL(dj_f32c_kernel<KID>, grid, dim3(kBlock), 0, f->stream, (const double*)pos, ld,         \
-                           (const float4*)gs, (const float*)cut, (const double*)tbox, np, delta, chunk, part);   \
+                           (const float4*)gs, (const float*)cut, (const double*)tbox, np, delta, part);          \
         hipLaunchKernelGGL(dj_finalize_kernel, dim3(nb), dim3(kBlock), 0, f->stream, (const double*)part,         \
                            (int)nchunk, np, dj);                                                                 \
         hipLaunchKernelGGL(de_f32c_kernel<KID>, grid, dim3(kBlock), 0, f->stream, (const double*)pos,             \
                            (const double*)J, (const double*)dj, ld, (const float4*)gz, (const float*)cut,         \
-                           (const double*)tbox, np, (float)alpha, transposed, chunk, part);                      \
+                           (const double*)tbox, np, (float)alpha, transposed, part);                             \
         hipLaunchKernelGGL(de_finalize_kernel, dim3(nb), dim3(kBlock), 0, f->stream, (const double*)part,         \
                            (int)nchunk, (const double*)J, (const double*)dj, ld, np, transposed, de);           \
         break;

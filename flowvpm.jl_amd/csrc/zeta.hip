@@ -54,7 +54,7 @@ __global__ __launch_bounds__(kBlock) void zeta_f32c_kernel(const double* __restr
                                                            const float4* __restrict__ gz,
                                                            const float2* __restrict__ bc,
                                                            const double* __restrict__ tbox, int64_t np,
-                                                           int64_t chunk, double* __restrict__ part, int64_t pld)
+                                                           double* __restrict__ part, int64_t pld)
 {
     __shared__ float4 lp[kTile];   // s'_hi x, y, z, cut
     __shared__ float4 lg[kTile];   // Gamma x, y, z, b
@@ -81,16 +81,14 @@ __global__ __launch_bounds__(kBlock) void zeta_f32c_kernel(const double* __restr
     block_box(box, wb, blo, bhi);
     const double org[3] = {ox, oy, oz};
 
-    const int64_t sb = by * chunk;
-    const int64_t se = min(sb + chunk, np);
     float sum[3] = {0.f, 0.f, 0.f}, err[3] = {0.f, 0.f, 0.f};
     __shared__ int nlist[kBlock];
     __shared__ int ncnt[kBlock / 64];
-    NearTiles near(tbox, sb / kTile, (se + kTile - 1) / kTile, org, blo, bhi, 1.0001f, nlist, ncnt);
+    NearTiles near(tbox, by, (np + kTile - 1) / kTile, gridDim.y, org, blo, bhi, 1.0001f, nlist, ncnt);
     for (int64_t tile; (tile = near.next()) >= 0;) {
         const int64_t base = tile * kTile;
         const int64_t j = base + tid;
-        const int n = (int)min((int64_t)kTile, se - base);
+        const int n = (int)min((int64_t)kTile, np - base);
         __syncthreads();
         if (tid < n) {
             const float4 g = gz[j];
@@ -228,12 +226,12 @@ int launch_zeta(vpm_field f, int kernel, int precision)
     const int64_t ld = f->cap;
     int rc;
     const unsigned nbt = (unsigned)((np + kBlock - 1) / kBlock);
-    // source splits, chunks of whole tiles: enough blocks to fill the chip,
-    // and up to 32 chunks of at least 16 tiles.  Near-field work per block is
-    // uneven (a block whose targets straddle a jump of the sort order reaches
-    // most tiles and finishes last); the chunks spread such a block's tiles
-    // over that many blocks.  At N = 2^20 on the jet column: 21 ms with one
-    // chunk, 12.4 with 8, 8.6 with 16, 6.6 with 32.
+    // source splits: enough blocks to fill the chip, and up to 32 (every K-th
+    // tile; contiguous chunks in FP64).  Near-field work per block is uneven (a
+    // block whose targets straddle a jump of the sort order reaches most tiles
+    // and finishes last); the splits spread such a block's tiles over that many
+    // blocks.  At N = 2^20 on the jet column with contiguous splits: 21 ms with
+    // one, 12.4 with 8, 8.6 with 16, 6.6 with 32.
     const int64_t tiles = (np + kTile - 1) / kTile;
     const int64_t k_fill = std::min<int64_t>((2560 + nbt - 1) / nbt, tiles);
     const int64_t k_spread = std::min<int64_t>(32, tiles / 16);
@@ -279,7 +277,7 @@ int launch_zeta(vpm_field f, int kernel, int precision)
                            (const double*)pos, ld, (const float*)bc + 1, np, tbox);                            \
         timing_begin(f);                                                                                       \
         hipLaunchKernelGGL(zeta_f32c_kernel<KID>, grid, dim3(kBlock), 0, f->stream, (const double*)pos, ld,     \
-                           (const float4*)gz, (const float2*)bc, (const double*)tbox, np, chunk, part, np);  \
+                           (const float4*)gz, (const float2*)bc, (const double*)tbox, np, part, np);  \
         break;
             VPM_Z32(VPM_KERNEL_GAUSSIAN) VPM_Z32(VPM_KERNEL_GAUSSIANERF) VPM_Z32(VPM_KERNEL_WINCKELMANS)
 #undef VPM_Z32
