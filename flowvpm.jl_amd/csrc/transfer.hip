@@ -4,14 +4,19 @@
 // The caller's array is pageable, so the runtime copies through a staging
 // buffer of its own on one thread, and a row range was then scattered on one
 // more pass: 28 ms for the 33 rows of 262,144 particles (69 MB), 70 ms for the
-// 15 rows of 2^20 -- for kernels that run in 1.5 and 350 ms.  Here a field
-// keeps a ring of kSlots pinned pieces of 1-4 MiB: the device copies (or
-// gathers rows) into one piece while host threads move another.  The ring
-// belongs to the field; row ranges need no device buffer (the gather writes
-// the pinned piece itself).
+// 15 rows of 2^20 -- for kernels that run in 1.5 and 350 ms.  Here a transfer
+// runs through a ring of kSlots pinned pieces of 1-4 MiB: the device copies
+// (or gathers rows) into one piece while host threads move another.  Row
+// ranges need no device buffer (the gather writes the pinned piece itself).
+//
+// Pinning a ring takes 0.2-2 ms, so rings outlive a transfer: a transfer takes
+// an idle one and gives it back when its stream has passed it.  At most
+// kIdleRings (12 MiB each) are kept, and none once the last field is gone.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
+#include <vector>
 
 #include "host_team.h"
 #include "vpm_internal.h"
@@ -44,6 +49,57 @@ __global__ __launch_bounds__(kBlock) void gather_rows_kernel(const double* __res
 
 namespace {
 
+constexpr size_t kIdleRings = 4;
+std::mutex g_ring_mu;
+std::vector<DevBuf> g_idle;      // guarded by g_ring_mu
+int64_t g_fields = 0;            // live fields
+
+// A ring for one transfer; nothing of it is in flight when it is destroyed.
+struct Ring {
+    DevBuf b;
+    ~Ring()
+    {
+        if (!b.p) return;
+        {
+            std::lock_guard<std::mutex> lk(g_ring_mu);
+            if (g_fields > 0 && g_idle.size() < g_idle.capacity()) {
+                g_idle.push_back(b);
+                return;
+            }
+        }
+        (void)hipHostFree(b.p);
+    }
+    int take(size_t bytes)
+    {
+        {
+            std::lock_guard<std::mutex> lk(g_ring_mu);
+            for (DevBuf& i : g_idle) {
+                if (i.bytes < bytes) continue;
+                b = i;
+                i = g_idle.back();
+                g_idle.pop_back();
+                return VPM_OK;
+            }
+            if (g_idle.size() == kIdleRings) {   // all too small: the new one takes a place
+                b = g_idle.back();
+                g_idle.pop_back();
+            }
+        }
+        if (b.p) {
+            (void)hipHostFree(b.p);
+            b = DevBuf();
+        }
+        const size_t want = std::max(bytes, (size_t)kSlots << 20);
+        const hipError_t e = hipHostMalloc(&b.p, want, hipHostMallocPortable);
+        if (e != hipSuccess) {
+            b.p = nullptr;
+            return hip_fail(e, "hipHostMalloc(transfer ring)");
+        }
+        b.bytes = want;
+        return VPM_OK;
+    }
+};
+
 // Events of the pieces in flight, for one call.
 struct Events {
     hipEvent_t ev[kSlots] = {};
@@ -70,6 +126,21 @@ void share(int64_t count, int w, int n, int64_t& a, int64_t& b)
 }
 
 }  // namespace
+
+int transfer_field(int change)
+{
+    std::vector<DevBuf> freed;
+    try {
+        std::lock_guard<std::mutex> lk(g_ring_mu);
+        if (change > 0) g_idle.reserve(kIdleRings);
+        g_fields += change;
+        if (g_fields == 0) freed.swap(g_idle);
+    } catch (const std::exception&) {
+        return fail(VPM_ENOMEM, "transfer rings");
+    }
+    for (DevBuf& b : freed) (void)hipHostFree(b.p);
+    return VPM_OK;
+}
 
 int check_records(const double* p, int64_t np)
 {
@@ -110,7 +181,8 @@ int upload_records(vpm_field f, const double* src, int64_t first, int64_t np)
     const int64_t per = std::min<int64_t>(np, (int64_t)(piece_bytes(rec * (size_t)np) / rec));
     const int64_t pieces = (np + per - 1) / per;
     const int slots = (int)std::min<int64_t>(kSlots, pieces);
-    if (int rc = ensure_pinned(f->ring, (size_t)slots * per * rec)) return rc;
+    Ring ring;
+    if (int rc = ring.take((size_t)slots * per * rec)) return rc;
     Events ev;
     if (int rc = ev.make(pieces > kSlots ? slots : 0)) return rc;
     HostTeam team(team_size(rec * (size_t)np));
@@ -118,7 +190,7 @@ int upload_records(vpm_field f, const double* src, int64_t first, int64_t np)
     for (int64_t k = 0; k < pieces && !rc; ++k) {
         const int s = (int)(k % slots);
         const int64_t a = k * per, n = std::min(per, np - a);
-        char* slot = (char*)f->ring.p + (size_t)s * per * rec;
+        char* slot = (char*)ring.b.p + (size_t)s * per * rec;
         hipError_t e = k >= slots ? hipEventSynchronize(ev.ev[s]) : hipSuccess;
         if (e != hipSuccess) { rc = hip_fail(e, "hipEventSynchronize"); break; }
         team.run([&](int w, int m) {
@@ -142,13 +214,14 @@ int download_rows(vpm_field f, double* dst, int64_t np, int row0, int row1)
     const int64_t per = std::min<int64_t>(np, (int64_t)(piece_bytes(rec * (size_t)np) / rec));
     const int64_t pieces = (np + per - 1) / per;
     const int slots = (int)std::min<int64_t>(kSlots, pieces);
-    if (int rc = ensure_pinned(f->ring, (size_t)slots * per * rec)) return rc;
+    Ring ring;
+    if (int rc = ring.take((size_t)slots * per * rec)) return rc;
     Events ev;
     if (int rc = ev.make(pieces > 1 ? slots : 0)) return rc;
     const auto issue = [&](int64_t k) -> int {
         const int s = (int)(k % slots);
         const int64_t a = k * per, n = std::min(per, np - a);
-        double* slot = (double*)((char*)f->ring.p + (size_t)s * per * rec);
+        double* slot = (double*)((char*)ring.b.p + (size_t)s * per * rec);
         hipError_t e;
         if (nr == NF) {
             e = hipMemcpyAsync(slot, f->P + a * NF, rec * (size_t)n, hipMemcpyDeviceToHost, f->stream);
@@ -170,7 +243,7 @@ int download_rows(vpm_field f, double* dst, int64_t np, int row0, int row1)
         const hipError_t e = ev.ev[s] ? hipEventSynchronize(ev.ev[s]) : hipStreamSynchronize(f->stream);
         if (e != hipSuccess) { rc = hip_fail(e, "particle download"); break; }
         const int64_t a = k * per, n = std::min(per, np - a);
-        const char* slot = (const char*)f->ring.p + (size_t)s * per * rec;
+        const char* slot = (const char*)ring.b.p + (size_t)s * per * rec;
         team.run([&](int w, int m) {
             int64_t b, c;
             share(n, w, m, b, c);

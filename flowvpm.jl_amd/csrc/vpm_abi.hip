@@ -252,6 +252,14 @@ int vpm_create(int device, int64_t maxparticles, vpm_field* out)
         delete f;
         return rc;
     }
+    if (int rc = transfer_field(1)) {
+        (void)hipFree(f->P);
+        (void)hipStreamDestroy(f->stream);
+        (void)hipEventDestroy(f->ev0);
+        (void)hipEventDestroy(f->ev1);
+        delete f;
+        return rc;
+    }
     *out = f;
     return VPM_OK;
 }
@@ -267,11 +275,9 @@ int vpm_destroy(vpm_field f)
                           &f->iota, &f->sorttmp, &f->bbox, &f->flag, &f->adj, &f->rng, &f->bar,
                           &f->lrec};
         for (DevBuf* b : bufs) release(*b);
-        for (DevBuf* b : {&f->hstage, &f->ring}) {
-            if (b->p) (void)hipHostFree(b->p);
-            b->p = nullptr;
-            b->bytes = 0;
-        }
+        if (f->hstage.p) (void)hipHostFree(f->hstage.p);
+        f->hstage.p = nullptr;
+        f->hstage.bytes = 0;
         for (vpm_tape t : f->tapes) {   // detach: the tape stays valid only for vpm_tape_destroy
             release(t->rec);
             t->f = nullptr;
@@ -288,6 +294,7 @@ int vpm_destroy(vpm_field f)
         if (f->ev0) (void)hipEventDestroy(f->ev0);
         if (f->ev1) (void)hipEventDestroy(f->ev1);
         if (f->stream) (void)hipStreamDestroy(f->stream);
+        (void)transfer_field(-1);
     }
     delete f;
     return VPM_OK;

@@ -85,7 +85,6 @@ struct vpm_field_s {
     vpm::DevBuf adj;                 // adjoint / E_str staging scratch
     vpm::DevBuf rng;                 // leaf-pair range lists
     vpm::DevBuf bar;                 // cotangent records of the step adjoint
-    vpm::DevBuf ring;                // pinned pieces of particle transfers (transfer.hip)
     vpm::DevBuf lrec;                // E_str / zeta list-kernel source records
     vpm::DevBuf hstage;              // pinned host staging of range plans (hipHostMalloc)
     bool profiling = false;
@@ -213,6 +212,8 @@ int launch_sfs_delta(vpm_field f, int kernel, int transposed, double alpha, Orde
 // record with sigma <= 0 or a non-finite X, Gamma or sigma.  upload_records
 // fills records [first, first + np); download_rows writes rows [row0, row1) of
 // the first np records into a 46-stride array.  Both wait for the stream.
+// transfer_field(+1 / -1) counts the live fields (the rings go with the last).
+int transfer_field(int change);
 int check_records(const double* p, int64_t np);
 int upload_records(vpm_field f, const double* src, int64_t first, int64_t np);
 int download_rows(vpm_field f, double* dst, int64_t np, int row0, int row1);
