@@ -122,8 +122,9 @@ __global__ __launch_bounds__(kBlock) void estr_f32c_kernel(
     split_rel_e(pos[it], ox, tx, tlx);
     split_rel_e(pos[ld + it], oy, ty, tly);
     split_rel_e(pos[2 * ld + it], oz, tz, tlz);
+    const WaveBox box = wave_box(tx, ty, tz);
     float blo[3], bhi[3];
-    block_box(wave_box(tx, ty, tz), wb, blo, bhi);
+    block_box(box, wb, blo, bhi);
     const double org[3] = {ox, oy, oz};
 
     float sum[6], err[6];
@@ -171,42 +172,64 @@ __global__ __launch_bounds__(kBlock) void estr_f32c_kernel(
         lq[tid] = q;
         ll[tid] = l;
         __syncthreads();
-        // fold into the compensated sums every 32 sources: E_str sums cancel
-        // strongly, so the FP32 tile sums are kept short
-        for (int s0 = 0; s0 < kTile; s0 += 32) {
-            float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-            for (int s = s0; s < s0 + 32; ++s) {
-                const float4 a = lp[s];
-                const float4 c = lq[s];
-                float dx = tx - a.x, dy = ty - a.y, dz = tz - a.z;
-                float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-                if (__any(r2 < c.w)) {
-                    const float4 lo = ll[s];
-                    const float4 b = lg[s];
-                    dx += tlx - lo.x;
-                    dy += tly - lo.y;
-                    dz += tlz - lo.z;
+        // The candidates of each 64 sources by one ballot; a fold into the
+        // compensated sums every 32 sources (E_str sums cancel strongly, so
+        // the FP32 sums are kept short), and none where no candidate was.
+        const int lane = tid & 63;
+#pragma unroll
+        for (int g0 = 0; g0 < kTile; g0 += 64) {
+            const float4 a0 = lp[g0 + lane];
+            const uint64_t cand = box_mask(box, a0.x, a0.y, a0.z, lq[g0 + lane].w, true);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                uint32_t m = (uint32_t)(cand >> (32 * h));
+                if (m == 0) continue;
+                float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                while (m) {
+                    // two candidates at a time, so that their loads and
+                    // exponentials overlap (the last one alone: twice the
+                    // same, the second with zeta = 0)
+                    const int s = g0 + 32 * h + __builtin_ctz(m);
+                    m &= m - 1;
+                    const int u = m ? g0 + 32 * h + __builtin_ctz(m) : s;
+                    const bool two = m != 0;
+                    m &= m - 1;
+                    const float4 as = lp[s], cs = lq[s], au = lp[u], cu = lq[u];
+                    float dx = tx - as.x, dy = ty - as.y, dz = tz - as.z;
+                    float ex = tx - au.x, ey = ty - au.y, ez = tz - au.z;
+                    float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+                    float q2 = fmaf(ez, ez, fmaf(ey, ey, ex * ex));
+                    const bool ins = __any(r2 < cs.w), inu = two && __any(q2 < cu.w);
+                    if (!ins && !inu) continue;
+                    const float4 los = ll[s], lou = ll[u], bs = lg[s], bu = lg[u];
+                    dx += tlx - los.x;
+                    dy += tly - los.y;
+                    dz += tlz - los.z;
+                    ex += tlx - lou.x;
+                    ey += tly - lou.y;
+                    ez += tlz - lou.z;
                     r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+                    q2 = fmaf(ez, ez, fmaf(ey, ey, ex * ex));
                     // the self pair adds (J_i - J_i)^T Gamma_i = 0 exactly in
                     // the reference, but the factored form would add it as
                     // zeta(0) J'_i^T Gamma_i twice with opposite signs
-                    const float z = base + s == i ? 0.f : zeta_sig<K>(r2, a.w, b.w);
-                    acc[0] = fmaf(z, b.x, acc[0]);
-                    acc[1] = fmaf(z, b.y, acc[1]);
-                    acc[2] = fmaf(z, b.z, acc[2]);
-                    acc[3] = fmaf(z, c.x, acc[3]);
-                    acc[4] = fmaf(z, c.y, acc[4]);
-                    acc[5] = fmaf(z, c.z, acc[5]);
+                    const float zs = !ins || base + s == i ? 0.f : zeta_sig<K>(r2, as.w, bs.w);
+                    const float zu = !inu || base + u == i ? 0.f : zeta_sig<K>(q2, au.w, bu.w);
+                    acc[0] = fmaf(zu, bu.x, fmaf(zs, bs.x, acc[0]));
+                    acc[1] = fmaf(zu, bu.y, fmaf(zs, bs.y, acc[1]));
+                    acc[2] = fmaf(zu, bu.z, fmaf(zs, bs.z, acc[2]));
+                    acc[3] = fmaf(zu, cu.x, fmaf(zs, cs.x, acc[3]));
+                    acc[4] = fmaf(zu, cu.y, fmaf(zs, cs.y, acc[4]));
+                    acc[5] = fmaf(zu, cu.z, fmaf(zs, cs.z, acc[5]));
                 }
-            }
 #pragma unroll
-            for (int c = 0; c < 6; ++c) {
-                const float x = acc[c];
-                const float t = sum[c] + x;
-                const float bp = t - sum[c];
-                err[c] += (sum[c] - (t - bp)) + (x - bp);
-                sum[c] = t;
+                for (int c = 0; c < 6; ++c) {
+                    const float x = acc[c];
+                    const float t = sum[c] + x;
+                    const float bp = t - sum[c];
+                    err[c] += (sum[c] - (t - bp)) + (x - bp);
+                    sum[c] = t;
+                }
             }
         }
     }

@@ -848,6 +848,18 @@ __device__ __forceinline__ float tile_gap2(const double* __restrict__ T, const d
     return g2;
 }
 
+// The sources of a 64-source group within their cut of the wave's target box
+// (one per lane: s'_hi and the cut; ok: a source at all).  As above, the box
+// distance never exceeds a target's FP32 hi distance, so a source outside this
+// mask is beyond its cut for every target.
+__device__ __forceinline__ uint64_t box_mask(const WaveBox& box, float x, float y, float z, float cut, bool ok)
+{
+    const float ex = fmaxf(fmaxf(box.lo[0] - x, x - box.hi[0]), 0.f);
+    const float ey = fmaxf(fmaxf(box.lo[1] - y, y - box.hi[1]), 0.f);
+    const float ez = fmaxf(fmaxf(box.lo[2] - z, z - box.hi[2]), 0.f);
+    return __ballot(ok && fmaf(ez, ez, fmaf(ey, ey, ex * ex)) < cut);
+}
+
 // The near tiles among t0, t0 + step, ... below t1 for a block, in ascending
 // order: kBlock tiles are tested at once (one per thread, independent loads), the near ones are
 // compacted into the __shared__ list, and next() walks the list.  A tile is

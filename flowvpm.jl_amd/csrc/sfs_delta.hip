@@ -73,11 +73,10 @@ __device__ __forceinline__ void delta_gk(float q, float delta, float& dg, float&
     dk = w * (kGlW0 * (k0 + k2) + kGlW1 * k1);
 }
 
-// zeta_s(r) = zeta(r/s)/s^3 and -d/ds of it, at width s (z0 = zeta(0) scale)
+// zeta_s(r) = zeta(r/s)/s^3 and -d/ds of it, at width s (si = 1/s)
 template <int K>
-__device__ __forceinline__ void zeta_and_rate(float r2, float s, float& z, float& rate)
+__device__ __forceinline__ void zeta_and_rate(float r2, float si, float& z, float& rate)
 {
-    const float si = 1.f / s;
     const float s3 = si * si * si;
     const float q2 = r2 * si * si;
     if constexpr (K == VPM_KERNEL_GAUSSIANERF) {
@@ -286,6 +285,7 @@ __global__ __launch_bounds__(kBlock) void de_f32c_kernel(const double* __restric
     __shared__ float4 l1[kTile];    // S(J'_j, Gamma_j)
     __shared__ float4 l2[kTile];    // S(dJ'_j, Gamma_j)
     __shared__ float4 ll[kTile];    // s'_lo
+    __shared__ float4 lw[kTile];    // 1/width at alpha sigma and the three points
     __shared__ float wb[kBlock / 64][6];
     const int tid = threadIdx.x;
     const int64_t i = (int64_t)blockIdx.x * kBlock + tid;
@@ -299,8 +299,9 @@ __global__ __launch_bounds__(kBlock) void de_f32c_kernel(const double* __restric
     split_rel(pos[it], ox, tx, tlx);
     split_rel(pos[ld + it], oy, ty, tly);
     split_rel(pos[2 * ld + it], oz, tz, tlz);
+    const WaveBox box = wave_box(tx, ty, tz);
     float blo[3], bhi[3];
-    block_box(wave_box(tx, ty, tz), wb, blo, bhi);
+    block_box(box, wb, blo, bhi);
     const double org[3] = {ox, oy, oz};
     float sum[12], err[12];
 #pragma unroll
@@ -340,6 +341,11 @@ __global__ __launch_bounds__(kBlock) void de_f32c_kernel(const double* __restric
                                  (float)(dJp[1] * G0 + dJp[4] * G1 + dJp[7] * G2),
                                  (float)(dJp[2] * G0 + dJp[5] * G1 + dJp[8] * G2), 0.f);
             }
+            // 1/s at the test width and at the Gauss-Legendre points between
+            // it and the source's own (a correctly rounded division takes ten
+            // instructions: here once per source instead of per pair)
+            const float st = alpha * g.w, w = oma * g.w;
+            lw[tid] = make_float4(1.f / st, 1.f / fmaf(w, kGlX0, st), 1.f / fmaf(w, kGlX1, st), 1.f / fmaf(w, kGlX2, st));
             lp[tid] = p;
             lg[tid] = make_float4(g.x, g.y, g.z, scut[j]);
             l1[tid] = s1;
@@ -347,58 +353,69 @@ __global__ __launch_bounds__(kBlock) void de_f32c_kernel(const double* __restric
             ll[tid] = l;
         }
         __syncthreads();
-        for (int s0 = 0; s0 < n; s0 += 32) {
-            const int s1e = min(s0 + 32, n);
-            float acc[12];
+        // candidates by one ballot per 64 sources, a fold every 32, as in estr.hip
+        const int lane = tid & 63;
 #pragma unroll
-            for (int c = 0; c < 12; ++c) acc[c] = 0.f;
-            for (int s = s0; s < s1e; ++s) {
-                const float4 a = lp[s];
-                const float4 g = lg[s];
-                float dx = tx - a.x, dy = ty - a.y, dz = tz - a.z;
-                float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-                if (__any(r2 < g.w && a.w > 0.f)) {
-                    if (!(a.w > 0.f)) continue;   // static source: no E_str term
-                    const float4 lo = ll[s];
-                    dx += tlx - lo.x;
-                    dy += tly - lo.y;
-                    dz += tlz - lo.z;
-                    r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-                    // dzeta = zeta_{alpha sigma} - zeta_sigma = int_{alpha sigma}^{sigma} rate(s) ds
-                    const float sg = a.w, w = oma * sg;
-                    float zt, r0, r1, r2v, z_;
-                    zeta_and_rate<K>(r2, alpha * sg, zt, r0);
-                    zeta_and_rate<K>(r2, fmaf(w, kGlX1, alpha * sg), z_, r1);
-                    zeta_and_rate<K>(r2, fmaf(w, kGlX2, alpha * sg), z_, r2v);
-                    float rq;
-                    zeta_and_rate<K>(r2, fmaf(w, kGlX0, alpha * sg), z_, rq);
-                    float dz_ = w * (kGlW0 * (rq + r2v) + kGlW1 * r1);
-                    // the self pair is exactly zero in the reference ((J_i -
-                    // J_i) and (dJ_i - dJ_i)); the factored form would add it
-                    // as cancelling terms
-                    if (base + s == i) { dz_ = 0.f; zt = 0.f; }
-                    const float4 c1 = l1[s], c2 = l2[s];
-                    acc[0] = fmaf(dz_, g.x, acc[0]);
-                    acc[1] = fmaf(dz_, g.y, acc[1]);
-                    acc[2] = fmaf(dz_, g.z, acc[2]);
-                    acc[3] = fmaf(dz_, c1.x, acc[3]);
-                    acc[4] = fmaf(dz_, c1.y, acc[4]);
-                    acc[5] = fmaf(dz_, c1.z, acc[5]);
-                    acc[6] = fmaf(zt, g.x, acc[6]);
-                    acc[7] = fmaf(zt, g.y, acc[7]);
-                    acc[8] = fmaf(zt, g.z, acc[8]);
-                    acc[9] = fmaf(zt, c2.x, acc[9]);
-                    acc[10] = fmaf(zt, c2.y, acc[10]);
-                    acc[11] = fmaf(zt, c2.z, acc[11]);
+        for (int g0 = 0; g0 < kTile; g0 += 64) {
+            const float4 a0 = lp[g0 + lane];
+            const uint64_t cand = box_mask(box, a0.x, a0.y, a0.z, lg[g0 + lane].w, g0 + lane < n && a0.w > 0.f);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                uint32_t m = (uint32_t)(cand >> (32 * h));   // static sources (a.w = 0) have no E_str term
+                if (m == 0) continue;
+                float acc[12];
+#pragma unroll
+                for (int c = 0; c < 12; ++c) acc[c] = 0.f;
+                while (m) {
+                    const int s = g0 + 32 * h + __builtin_ctz(m);
+                    m &= m - 1;
+                    const float4 a = lp[s];
+                    const float4 g = lg[s];
+                    float dx = tx - a.x, dy = ty - a.y, dz = tz - a.z;
+                    float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+                    if (__any(r2 < g.w)) {
+                        const float4 lo = ll[s];
+                        dx += tlx - lo.x;
+                        dy += tly - lo.y;
+                        dz += tlz - lo.z;
+                        r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+                        // dzeta = zeta_{alpha sigma} - zeta_sigma = int_{alpha sigma}^{sigma} rate(s) ds
+                        const float w = oma * a.w;
+                        const float4 si = lw[s];
+                        float zt, r0, r1, r2v, z_;
+                        zeta_and_rate<K>(r2, si.x, zt, r0);
+                        zeta_and_rate<K>(r2, si.z, z_, r1);
+                        zeta_and_rate<K>(r2, si.w, z_, r2v);
+                        float rq;
+                        zeta_and_rate<K>(r2, si.y, z_, rq);
+                        float dz_ = w * (kGlW0 * (rq + r2v) + kGlW1 * r1);
+                        // the self pair is exactly zero in the reference ((J_i -
+                        // J_i) and (dJ_i - dJ_i)); the factored form would add it
+                        // as cancelling terms
+                        if (base + s == i) { dz_ = 0.f; zt = 0.f; }
+                        const float4 c1 = l1[s], c2 = l2[s];
+                        acc[0] = fmaf(dz_, g.x, acc[0]);
+                        acc[1] = fmaf(dz_, g.y, acc[1]);
+                        acc[2] = fmaf(dz_, g.z, acc[2]);
+                        acc[3] = fmaf(dz_, c1.x, acc[3]);
+                        acc[4] = fmaf(dz_, c1.y, acc[4]);
+                        acc[5] = fmaf(dz_, c1.z, acc[5]);
+                        acc[6] = fmaf(zt, g.x, acc[6]);
+                        acc[7] = fmaf(zt, g.y, acc[7]);
+                        acc[8] = fmaf(zt, g.z, acc[8]);
+                        acc[9] = fmaf(zt, c2.x, acc[9]);
+                        acc[10] = fmaf(zt, c2.y, acc[10]);
+                        acc[11] = fmaf(zt, c2.z, acc[11]);
+                    }
                 }
-            }
 #pragma unroll
-            for (int c = 0; c < 12; ++c) {
-                const float x = acc[c];
-                const float t = sum[c] + x;
-                const float bp = t - sum[c];
-                err[c] += (sum[c] - (t - bp)) + (x - bp);
-                sum[c] = t;
+                for (int c = 0; c < 12; ++c) {
+                    const float x = acc[c];
+                    const float t = sum[c] + x;
+                    const float bp = t - sum[c];
+                    err[c] += (sum[c] - (t - bp)) + (x - bp);
+                    sum[c] = t;
+                }
             }
         }
     }
