@@ -538,6 +538,67 @@ __device__ __forceinline__ double rsqrt_pos(double x)
     return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
+#pragma clang fp contract(off)
+// r^2 beyond which pair_f64 with g = 1 and dg/dr = 0 gives the same bits
+// (never, where the kernel has no such r^2 or sigma is out of range):
+//  * Gaussian-erf, q >= 10: q/sqrt2 > 6, where custom_erf64 is 1, minus
+//    sqrt(2/pi) q e^{-q^2/2} < 2e-21, rounds to 1; dg/(sigma r) is below
+//    6e-20 of the 3 g / r^2 it is added to;
+//  * Gaussian, q^2 >= 13: e^{-q^3} < 5e-21, and 3e-19 of 3 g / r^2.
+// With sigma in [1e-100, 1e100] and r^2 below kLitR2Max nothing in those
+// expressions is a NaN that leaving them out would hide.
+// A far pair is 76 FP64 instructions instead of 190 (exp, erf's branch test,
+// a square root and four divisions).  U/J of 40,000 leapfrog particles 10.8 ->
+// 6.0 ms, of 16,384 2.05 -> 1.57 ms (24 % of the (wave, source) pairs are near
+// and run every branch of erf that a lane needs); a 16,384 cloud in random
+// storage order, 4 % of its pairs far, 2.97 -> 2.89 ms.
+constexpr double kLitR2Max = 1e200;
+template <int K>
+__device__ __forceinline__ double lit_cut64(double sigma)
+{
+    const bool cheap = K == VPM_KERNEL_GAUSSIANERF || K == VPM_KERNEL_GAUSSIAN;
+    if (!cheap || !(sigma >= 1e-100 && sigma <= 1e100)) return DBL_MAX;
+    return (K == VPM_KERNEL_GAUSSIANERF ? 100.0001 : 13.0001) * sigma * sigma;
+}
+
+// pair_f64 beyond lit_cut64.  The square root and the two divisions take one
+// reciprocal square root, each rounded once more from its exact remainder
+// (P. Markstein, "Computation of elementary functions on the IA-64", 2000):
+// the value before that rounding is off by less than 2^-100, so it is the
+// correctly rounded one but for about one operand in 2^47.
+__device__ __forceinline__ void pair_f64_lit_far(double dx, double dy, double dz, double r2, const double4 b,
+                                                 double (&acc)[kAccF64])
+{
+    const double ri = rsqrt_pos(r2);
+    const double r0 = r2 * ri;
+    const double r = fma(fma(-r0, r0, r2), 0.5 * ri, r0);   // sqrt(r2)
+    const double r3 = r2 * r;
+    const double y2 = ri * ri, y3 = y2 * ri;
+    const double r2inv = fma(fma(-r2, y2, 1.0), y2, y2);
+    const double r3inv = fma(fma(-r3, y3, 1.0), y3, y3);    // 1 / (r2 r)
+    const double t = 3.0 * r2inv;
+    const double aux = -fma(fma(-r2, t, 3.0), r2inv, t);    // -3 / r2
+    const double c = -kConst4 * r3inv;                      // also aux2
+    const double crss1 = c * (dy * b.z - dz * b.y);
+    const double crss2 = c * (dz * b.x - dx * b.z);
+    const double crss3 = c * (dx * b.y - dy * b.x);
+    acc[0] += crss1;
+    acc[1] += crss2;
+    acc[2] += crss3;
+    const double h1 = aux * crss1, h2 = aux * crss2, h3 = aux * crss3;
+    const double wx = c * b.x, wy = c * b.y, wz = c * b.z;
+    acc[3] += h1 * dx;
+    acc[4] += h2 * dx - wz;
+    acc[5] += h3 * dx + wy;
+    acc[6] += h1 * dy + wz;
+    acc[7] += h2 * dy;
+    acc[8] += h3 * dy - wx;
+    acc[9] += h1 * dz - wy;
+    acc[10] += h2 * dz + wx;
+    acc[11] += h3 * dz;
+}
+#pragma clang fp contract(on)
+
 // accum_pair in FP64 (the 14 sums of add_f32c_to_record)
 __device__ __forceinline__ void accum_pair64(double dx, double dy, double dz, double Fp, double Hpp,
                                              const double4 b, double (&acc)[kAccF32])

@@ -29,7 +29,9 @@
 //
 // F64: the reference's FP64 pair arithmetic statement by statement
 // (fmm.jl:113-161, kernel.jl:45-84, custom_erf64 of gpu_erf.jl:159-191),
-// contraction off, sources in storage order.  This is the GPU FP64 oracle.
+// contraction off, sources in storage order; a source whose g and dg/dr are 1
+// and 0 to the last bit at every target of the wave skips both (lit_cut64).
+// This is the GPU FP64 oracle.
 #include <cfloat>
 #include <cstring>
 
@@ -116,12 +118,12 @@ __global__ __launch_bounds__(kBlock) void uj_f64_kernel(
     int64_t s0, int64_t s1, int64_t chunk, double* __restrict__ part, int64_t pld)
 {
     __shared__ double4 lpos[kTile];   // x, y, z, sigma
-    __shared__ double4 lgam[kTile];   // Gamma x, y, z
+    __shared__ double4 lgam[kTile];   // Gamma x, y, z, lit_cut64
 
     const int tid = threadIdx.x;
     const int64_t i = (int64_t)blockIdx.x * kBlock + tid;
     const bool active = i < nt;
-    const int64_t it = t0 + (active ? i : 0);
+    const int64_t it = t0 + min(i, nt - 1);
     const double tx = tpos[it], ty = tpos[tld + it], tz = tpos[2 * tld + it];
     const int64_t sb = s0 + (int64_t)blockIdx.y * chunk;
     const int64_t se = min(sb + chunk, s1);
@@ -137,10 +139,19 @@ __global__ __launch_bounds__(kBlock) void uj_f64_kernel(
         if (tid < n) {
             const double4 gg = sg[j];
             lpos[tid] = make_double4(spos[j], spos[sld + j], spos[2 * sld + j], gg.w);
-            lgam[tid] = make_double4(gg.x, gg.y, gg.z, 0.0);
+            lgam[tid] = make_double4(gg.x, gg.y, gg.z, lit_cut64<K>(gg.w));
         }
         __syncthreads();
-        for (int s = 0; s < n; ++s) pair_f64<K>(tx, ty, tz, lpos[s], lgam[s], acc);
+        for (int s = 0; s < n; ++s) {   // a run of far sources, then a near one
+            for (; s < n; ++s) {
+                const double4 a = lpos[s], b = lgam[s];
+                const double dx = tx - a.x, dy = ty - a.y, dz = tz - a.z;
+                const double r2 = dx * dx + dy * dy + dz * dz;
+                if (__any(!(r2 > b.w && r2 < kLitR2Max))) break;
+                pair_f64_lit_far(dx, dy, dz, r2, b, acc);
+            }
+            if (s < n) pair_f64<K>(tx, ty, tz, lpos[s], lgam[s], acc);
+        }
     }
     if (active) {
         double* out = part + (int64_t)blockIdx.y * kAccF64 * pld + i;
