@@ -282,6 +282,28 @@ __device__ __forceinline__ double zeta_ref(double r)
     }
 }
 
+// r^2 beyond which zeta_ref is exactly 0 (never, with sigma out of range):
+// e^-745.2 rounds to 0, past q = 39 for Gaussian-erf and q^2 = 83 for the
+// Gaussian; the singular kernel's zeta is nonzero at r = 0 only.  Skipping such
+// sources and dividing by sigma once per source: E_str of 40,000 leapfrog / jet
+// particles 5.4 -> 3.3 / 4.0 ms, of the 30,011 cloud (none skipped) 3.1 -> 2.9.
+template <int K>
+__device__ __forceinline__ double zeta_zero64(double sigma)
+{
+    if (K == VPM_KERNEL_WINCKELMANS || !(sigma >= 1e-100 && sigma <= 1e100)) return INFINITY;
+    return K == VPM_KERNEL_GAUSSIANERF ? 1521.0 * sigma * sigma : K == VPM_KERNEL_GAUSSIAN ? 83.0 * sigma * sigma : 0.0;
+}
+
+// Whether every |x| is below 1e100 (no infinity, no NaN)
+template <int N>
+__device__ __forceinline__ bool all_tame(const double* x)
+{
+    bool ok = true;
+#pragma unroll
+    for (int c = 0; c < N; ++c) ok &= fabs(x[c]) < 1e100;
+    return ok;
+}
+
 // One block per 256 targets (storage order) and source split (whole tiles);
 // sources in storage order.  With every source in one block, the 64 blocks of
 // 16,384 particles left three quarters of the chip idle.
@@ -289,17 +311,18 @@ template <int K>
 __global__ __launch_bounds__(kBlock) void estr_f64_kernel(const double* __restrict__ P, int64_t np, int transposed,
                                                           int64_t chunk, double* __restrict__ part, int64_t pld)
 {
-    __shared__ double lx[kTile][4];
-    __shared__ double lg[kTile][4];
+    __shared__ double lx[kTile][4];   // x, y, z, 1/sigma
+    __shared__ double lg[kTile][4];   // Gamma, r^2 beyond which the source adds exactly nothing
     __shared__ double lj[kTile][9];
     const int tid = threadIdx.x;
     const int64_t i = (int64_t)blockIdx.x * kBlock + tid;
-    const int64_t it = i < np ? i : 0;
+    const int64_t it = min(i, np - 1);
     const double* tr = P + it * NF;
     const double tx = tr[RX], ty = tr[RX + 1], tz = tr[RX + 2];
     double JT[9];
 #pragma unroll
     for (int c = 0; c < 9; ++c) JT[c] = tr[RJ + c];
+    const bool tame = !__any(!all_tame<9>(JT));
     double s1 = 0, s2 = 0, s3 = 0;
     const int64_t sb = (int64_t)blockIdx.y * chunk, se = min(sb + chunk, np);
     for (int64_t base = sb; base < se; base += kTile) {
@@ -307,16 +330,21 @@ __global__ __launch_bounds__(kBlock) void estr_f64_kernel(const double* __restri
         __syncthreads();
         if (tid < n) {
             const double* sr = P + (base + tid) * NF;
-            lx[tid][0] = sr[RX]; lx[tid][1] = sr[RX + 1]; lx[tid][2] = sr[RX + 2]; lx[tid][3] = sr[RSIG];
-            lg[tid][0] = sr[RG]; lg[tid][1] = sr[RG + 1]; lg[tid][2] = sr[RG + 2]; lg[tid][3] = sr[RSTATIC];
+            lx[tid][0] = sr[RX]; lx[tid][1] = sr[RX + 1]; lx[tid][2] = sr[RX + 2]; lx[tid][3] = 1.0 / sr[RSIG];
+            lg[tid][0] = sr[RG]; lg[tid][1] = sr[RG + 1]; lg[tid][2] = sr[RG + 2];
 #pragma unroll
             for (int c = 0; c < 9; ++c) lj[tid][c] = sr[RJ + c];
+            lg[tid][3] = sr[RSTATIC] != 0 ? -1.0
+                         : all_tame<3>(lg[tid]) && all_tame<9>(lj[tid]) ? zeta_zero64<K>(sr[RSIG]) : INFINITY;
         }
         __syncthreads();
         for (int s = 0; s < n; ++s) {
-            if (lg[s][3] != 0) continue;                    // static source
+            const double cut = lg[s][3];
+            if (cut < 0) continue;                          // static source
             const double dx = lx[s][0] - tx, dy = lx[s][1] - ty, dz = lx[s][2] - tz;
-            const double r = sqrt(dx * dx + dy * dy + dz * dz);
+            const double r2 = dx * dx + dy * dy + dz * dz;
+            if (tame && !__any(!(r2 > cut))) continue;      // zeta_sgm = 0
+            const double r = sqrt(r2);
             const double* JS = lj[s];
             const double* GS = lg[s];
             double S1, S2, S3;
@@ -329,7 +357,7 @@ __global__ __launch_bounds__(kBlock) void estr_f64_kernel(const double* __restri
                 S2 = (JT[1] - JS[1]) * GS[0] + (JT[4] - JS[4]) * GS[1] + (JT[7] - JS[7]) * GS[2];
                 S3 = (JT[2] - JS[2]) * GS[0] + (JT[5] - JS[5]) * GS[1] + (JT[8] - JS[8]) * GS[2];
             }
-            const double sigma_inv = 1.0 / lx[s][3];
+            const double sigma_inv = lx[s][3];
             const double zeta_sgm = zeta_ref<K>(r * sigma_inv) * sigma_inv * sigma_inv * sigma_inv;
             s1 += zeta_sgm * S1;
             s2 += zeta_sgm * S2;
