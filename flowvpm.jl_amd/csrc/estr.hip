@@ -102,7 +102,7 @@ template <int K>
 __global__ __launch_bounds__(kBlock) void estr_f32c_kernel(
     const double* __restrict__ pos, const double* __restrict__ J, int64_t ld,
     const float4* __restrict__ gz, const float2* __restrict__ bc, const double* __restrict__ tbox, int64_t np,
-    int transposed, double* __restrict__ part, int64_t pld)
+    int quarters, int transposed, double* __restrict__ part, int64_t pld)
 {
     __shared__ float4 lp[kTile];   // s'_hi x, y, z, a
     __shared__ float4 lg[kTile];   // Gamma x, y, z, b
@@ -133,12 +133,16 @@ __global__ __launch_bounds__(kBlock) void estr_f32c_kernel(
 
     __shared__ int nlist[kBlock];
     __shared__ int ncnt[kBlock / 64];
-    NearTiles near(tbox, blockIdx.y, (np + kTile - 1) / kTile, gridDim.y, org, blo, bhi, 1.0f, nlist, ncnt);
+    // quarters: a block takes 64 sources of each of its tiles
+    const int split = quarters ? blockIdx.y >> 2 : blockIdx.y;
+    const int gb = quarters ? (blockIdx.y & 3) * 64 : 0, ge = quarters ? gb + 64 : kTile;
+    NearTiles near(tbox, split, (np + kTile - 1) / kTile, quarters ? gridDim.y >> 2 : gridDim.y, org, blo, bhi, 1.0f,
+                   nlist, ncnt);
     for (int64_t tile; (tile = near.next()) >= 0;) {
         const int64_t base = tile * kTile;
         const int64_t j = base + tid;
         float4 p, g, q, l;
-        if (j < np) {
+        if (j < np && tid >= gb && tid < ge) {
             const float4 gg = gz[j];
             const float2 b = bc[j];
             split_rel_e(pos[j], ox, p.x, l.x);
@@ -176,8 +180,7 @@ __global__ __launch_bounds__(kBlock) void estr_f32c_kernel(
         // compensated sums every 32 sources (E_str sums cancel strongly, so
         // the FP32 sums are kept short), and none where no candidate was.
         const int lane = tid & 63;
-#pragma unroll
-        for (int g0 = 0; g0 < kTile; g0 += 64) {
+        for (int g0 = gb; g0 < ge; g0 += 64) {
             const float4 a0 = lp[g0 + lane];
             const uint64_t cand = box_mask(box, a0.x, a0.y, a0.z, lq[g0 + lane].w, true);
 #pragma unroll
@@ -560,6 +563,11 @@ static int64_t near_splits(int64_t np)
     return std::max<int64_t>({1, std::min<int64_t>((2560 + nb - 1) / nb, tiles), std::min<int64_t>(32, tiles / 16)});
 }
 
+// Most blocks of an F32C E_str launch whose tiles are split in quarters: E_str
+// of 1,000 / 3,001 / 5,000 particles 60 / 65 / 71 -> 36 / 42 / 60 us; at 8,000
+// (1,024 blocks) 73 -> 69, but Winckelmans, which skips nothing, 94 -> 100.
+static constexpr int64_t kQuarterBlocks = 512;
+
 int launch_estr_impl(vpm_field f, int kernel, int transposed, int precision, const uint32_t* perm)
 {
     const int64_t np = f->np;
@@ -569,9 +577,10 @@ int launch_estr_impl(vpm_field f, int kernel, int transposed, int precision, con
     // where the reference's (J_t - J_s) difference is exact: use FP64.
     if (precision == VPM_PREC_F64 || kernel == VPM_KERNEL_SINGULAR) {
         // 4,096 blocks of equal work (16 waves per SIMD)
-        const int64_t tiles = (np + kTile - 1) / kTile;
-        int64_t K = std::min<int64_t>(std::max<int64_t>(1, 4096 / nblk(np)), tiles);
-        const int64_t chunk = ((tiles + K - 1) / K) * kTile;
+        const int64_t grain = split_grain(nblk(np), np);
+        const int64_t steps = (np + grain - 1) / grain;
+        int64_t K = std::min<int64_t>(std::max<int64_t>(1, 4096 / nblk(np)), steps);
+        const int64_t chunk = ((steps + K - 1) / K) * grain;
         K = (np + chunk - 1) / chunk;
         if ((rc = ensure(f->part, sizeof(double) * 3 * (size_t)K * (size_t)np))) return rc;
         double* part = (double*)f->part.p;
@@ -618,12 +627,15 @@ int launch_estr_impl(vpm_field f, int kernel, int transposed, int precision, con
                        (const float*)bc + 1, np, tbox);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "pack_estr");
-    const int64_t K = near_splits(np);
+    int64_t K = near_splits(np);
+    // four blocks to a tile where every tile has its own and the chip is idle
+    const int quarters = K == (int64_t)ntile && K * nblk(np) <= kQuarterBlocks;
+    if (quarters) K *= 4;
     if ((rc = ensure(f->part, sizeof(double) * 6 * (size_t)K * (size_t)np))) return rc;
     double* part = (double*)f->part.p;
     timing_begin(f);
     switch (kernel) {
-#define VPM_ES(KID) case KID: hipLaunchKernelGGL(estr_f32c_kernel<KID>, dim3(nblk(np), (unsigned)K), dim3(kBlock), 0, f->stream, pos, J, ld, gz, bc, (const double*)tbox, np, transposed, part, np); break;
+#define VPM_ES(KID) case KID: hipLaunchKernelGGL(estr_f32c_kernel<KID>, dim3(nblk(np), (unsigned)K), dim3(kBlock), 0, f->stream, pos, J, ld, gz, bc, (const double*)tbox, np, quarters, transposed, part, np); break;
         VPM_ES(VPM_KERNEL_GAUSSIAN) VPM_ES(VPM_KERNEL_GAUSSIANERF) VPM_ES(VPM_KERNEL_WINCKELMANS)
 #undef VPM_ES
     default: return fail(VPM_EINVAL, "unknown kernel id");

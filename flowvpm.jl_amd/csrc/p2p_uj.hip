@@ -607,22 +607,41 @@ int stage_field(vpm_field f, int kernel, int precision, Order order, Staged& out
     return VPM_OK;
 }
 
+// Sources per step of a split's chunk: a whole tile, or a part of one where a
+// launch of nblk target blocks would leave the chip idle (a block of fewer
+// sources reads and writes as much per target, so no smaller than needed):
+// half a tile below 4,096 blocks, then halved until there are over 1,024.
+// U/J with 256 sources, and with this rule: ring of 100 51 -> 30 us, of 300
+// 88 -> 30, cloud of 1,000 88 -> 37, of 3,001 91 -> 57, of 12,000 219 -> 193;
+// 8,000 particles 128 -> 124 (64 sources: 137); FP64 of 2,000 leapfrog
+// particles 285 -> 79, far form 227 -> 73, of the 12,000 cloud 798 -> 524.  At
+// 4,096 blocks (16,384 particles) half a tile is no gain: 316 -> 320 us, FP64
+// 1,400 -> 1,639.
+int64_t split_grain(int64_t nblk, int64_t ns)
+{
+    int64_t g = kTile;
+    const auto blocks = [&] { return nblk * ((ns + g - 1) / g); };
+    if (blocks() < 4096) g = kTile / 2;
+    while (g > kTile / 16 && blocks() <= 1024) g /= 2;
+    return g;
+}
+
 // Number of source splits: about 32,768 blocks in all, chunks a multiple of
-// the tile.  Blocks differ in near-field work, and many short blocks balance
-// the CUs better than a few long ones: against 2,560 blocks, 32,768 run
-// 11-25 % faster from N = 32,768 to 262,144, and at N = 2^20 (K = 8 instead
-// of 1) 3-5 % faster; beyond that the gain is flat.  The FP64 partial sums
-// then take at most ~1 GB (K x 14 x 8 B per target).
+// split_grain.  Blocks differ in near-field work, and many short blocks
+// balance the CUs better than a few long ones: against 2,560 blocks, 32,768
+// run 11-25 % faster from N = 32,768 to 262,144, and at N = 2^20 (K = 8
+// instead of 1) 3-5 % faster; beyond that the gain is flat.  The FP64 partial
+// sums then take at most ~1 GB (K x 14 x 8 B per target).
 void choose_split(int64_t nt, int64_t ns, int64_t kmax, int64_t& K, int64_t& chunk)
 {
     const int64_t nblk = (nt + kBlock - 1) / kBlock;
     const int64_t want = 32768;
     K = std::max<int64_t>(1, (want + nblk - 1) / nblk);
     if (kmax > 0) K = std::min(K, kmax);
-    const int64_t tiles = std::max<int64_t>(1, (ns + kTile - 1) / kTile);
-    K = std::min(K, tiles);
-    const int64_t tiles_per = (tiles + K - 1) / K;
-    chunk = tiles_per * kTile;
+    const int64_t grain = split_grain(nblk, ns);
+    const int64_t steps = std::max<int64_t>(1, (ns + grain - 1) / grain);
+    K = std::min(K, steps);
+    chunk = ((steps + K - 1) / K) * grain;
     K = (ns + chunk - 1) / chunk;
     if (K < 1) K = 1;
 }

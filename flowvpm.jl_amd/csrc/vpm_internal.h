@@ -161,7 +161,9 @@ int launch_uj(vpm_field ft, const Staged& T, int64_t t0, int64_t nt,
               const Staged& S, int64_t s0, int64_t s1, int kernel, int precision,
               bool far, Arena* ar = nullptr, int64_t kmax = 0);
 // Source splits of an all-pairs launch over nt targets and ns sources (at
-// most kmax when kmax > 0): K chunks of `chunk` sources, a multiple of the tile.
+// most kmax when kmax > 0): K chunks of `chunk` sources, a multiple of
+// split_grain (a tile, or a part of one for small fields).
+int64_t split_grain(int64_t nblk, int64_t ns);
 void choose_split(int64_t nt, int64_t ns, int64_t kmax, int64_t& K, int64_t& chunk);
 // Scratch bytes of sort_field (temp storage of the radix sort included).
 int sort_scratch_bytes(vpm_field f, size_t& bytes);

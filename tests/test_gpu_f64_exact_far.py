@@ -41,9 +41,9 @@ def _hold(A, R, scale):
                                       ("singular", 10.0)])
 @pytest.mark.parametrize("n", [64, 65, 256])
 def test_uj_bits(vpm, kernel, q, n):
-    """One tile and one list item take the sources in the same order, so the
-    all-pairs kernel has the bits of the list kernel, which evaluates g and
-    dg/dr of every pair."""
+    """One source with strength at a time, so that no order of summation
+    matters: the all-pairs kernel has the bits of the list kernel, which
+    evaluates g and dg/dr of every pair."""
     X, G, S = _spread(n, q, n)
     for case in ("plain", "sigma out of range", "great strength", "great distance"):
         P = vpm.fields.make_particles(X, G, S)
@@ -53,12 +53,16 @@ def test_uj_bits(vpm, kernel, q, n):
             P[n // 2, 3] = 1e300
         elif case == "great distance":
             P[n // 2, 1] = 1e120
-        A, B = P.copy(), P.copy()
-        print(kernel, n, case, flush=True)
-        vpm.UJ_hip(A, kernel=kernel, precision="f64")
-        vpm.p2p_ranges(B, [0], [n], [0], [n], kernel=kernel, precision="f64")
-        assert np.array_equal(A[:, 9:24], B[:, 9:24], equal_nan=True), case
-        assert case != "plain" or np.all(np.isfinite(A[:, 9:24]))
+        for j in (0, 1, 2, 3, 5, n // 2, n - 1):
+            A = P.copy()
+            A[:, 3:6] = 0.0
+            A[j, 3:6] = P[j, 3:6]
+            B = A.copy()
+            print(kernel, n, case, j, flush=True)
+            vpm.UJ_hip(A, kernel=kernel, precision="f64")
+            vpm.p2p_ranges(B, [0], [n], [0], [n], kernel=kernel, precision="f64")
+            assert np.array_equal(A[:, 9:24], B[:, 9:24], equal_nan=True), (case, j)
+            assert case != "plain" or np.all(np.isfinite(A[:, 9:24]))
 
 
 @pytest.mark.parametrize("kernel,q", [("gaussianerf", 39.0), ("gaussian", 83 ** 0.5), ("winckelmans", 39.0),
