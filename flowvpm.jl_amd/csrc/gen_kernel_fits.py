@@ -31,6 +31,11 @@ harder:
 These are entire functions; the polynomials are weighted least-squares fits
 (relative error) at Chebyshev nodes, from 40-digit mpmath values.
 
+The FP64 far-form kernel takes phi1 and S in FP64, in t - 2 (t = q^2 in [0, 4])
+and w - 0.35 (w in [0.1, 0.5]); with E and phi1, phi0 = t phi1 + sqrt(2/pi) E/3
+without cancellation.  S's error is weighted by E w / (g - q g'/3), its share
+of H''.  Past q = 10 the fit is extrapolated to w = 0, where E < 2e-22.
+
     python gen_kernel_fits.py > kernel_fits.h
 """
 import mpmath as mp
@@ -106,6 +111,30 @@ def fit(f, a, b, deg, idx, n=256, absolute=False):
     return cf, err
 
 
+def fit64(f, a, b, c, deg, weight, n=80):
+    """Weighted least squares in 60 digits, in powers of x - c."""
+    with mp.workdps(60):
+        a, b, c = mp.mpf(a), mp.mpf(b), mp.mpf(c)
+        A, y = mp.matrix(n, deg + 1), mp.matrix(n, 1)
+        for i in range(n):
+            x = (mp.cos(mp.pi * (i + mp.mpf(0.5)) / n) * (b - a) + a + b) / 2
+            w = weight(x)
+            for k in range(deg + 1):
+                A[i, k] = w * (x - c) ** k
+            y[i] = w * f(x)
+        co = mp.lu_solve(A.T * A, A.T * y)
+        co = [float(co[k]) for k in range(deg + 1)]
+        xs = [a + (b - a) * i / 400 for i in range(401)]
+        err = max(abs(mp.polyval([mp.mpf(v) for v in co[::-1]], x - c) - f(x)) * weight(x) for x in xs)
+    return co, float(err)
+
+
+def emit64(name, coefs, err, var):
+    return ("// %s: degree %d in %s, max weighted error %.1e\n"
+            "static constexpr double %s[%d] = {%s};\n" % (name, len(coefs) - 1, var, err, name, len(coefs),
+                                                            ", ".join("%.17e" % v for v in coefs)))
+
+
 def emit(name, coefs, err, var):
     body = ", ".join("%.9ef" % float(c) for c in coefs)
     return ("// %s: degree %d in %s, max rel. error of FP32 Horner %.1e\n"
@@ -135,6 +164,18 @@ def main():
         out.append(emit(name, c, e, "u"))
     c, e = fit(gau_chi, 0.0, 1.0, 8, 0, absolute=True)
     out.append(emit("kGauChi", c, e, "u").replace("max rel. error", "max error / max|chi|"))
+    out.append("// FP64, Gaussian-erf: phi1 on t = q^2 in [0, 4], S on w = 1/q in [0.1, 0.5]")
+    out.append("static constexpr double kErf64TMax = 4.0, kErf64TMid = 2.0, kErf64WMid = 0.35;")
+    c, e = fit64(lambda t: erf_phi(t)[1], "1e-9", 4, 2, 14, lambda t: 1 / erf_phi(t)[1])
+    out.append(emit64("kErf64Phi1", c, e, "t - 2"))
+    c, e = fit64(lambda w: erfc_s(w)[0], "0.1", "0.5", "0.35", 13,
+                 lambda w: mp.exp(-1 / w ** 2 / 2) * w / (erf_phi(1 / w ** 2)[1] / w ** 5) + mp.mpf("1e-17"))
+    out.append(emit64("kErf64S", c, e, "w - 0.35"))
+    out.append("// e^x on |x| <= ln(2)/2, and ln 2 = hi + lo (hi of 32 bits: k hi is exact)")
+    hi = float(mp.floor(mp.log(2) * 2 ** 32) / 2 ** 32)
+    out.append("static constexpr double kLn2Hi = %.17e, kLn2Lo = %.17e;" % (hi, float(mp.log(2) - hi)))
+    c, e = fit64(mp.exp, "-0.3466", "0.3466", 0, 11, lambda x: mp.exp(-x))
+    out.append(emit64("kExp64", c, e, "x"))
     print("\n".join(out))
 
 

@@ -28,3 +28,16 @@ static constexpr float kGauPsi[8] = {5.000000000e-01f, -3.333333135e-01f, 1.2499
 // kGauChi: degree 8 in u, max error / max|chi| of FP32 Horner 2.7e-07
 static constexpr float kGauChi[9] = {-1.500000000e+00f, 4.000000000e+00f, -2.624999523e+00f, 9.999954700e-01f, -2.708097100e-01f, 5.707337335e-02f, -9.774587117e-03f, 1.329398714e-03f, -1.125588024e-04f};
 
+// FP64, Gaussian-erf: phi1 on t = q^2 in [0, 4], S on w = 1/q in [0.1, 0.5]
+static constexpr double kErf64TMax = 4.0, kErf64TMid = 2.0, kErf64WMid = 0.35;
+// kErf64Phi1: degree 14 in t - 2, max weighted error 1.9e-16
+static constexpr double kErf64Phi1[15] = {2.66676419900561158e-02, -8.87410862528015959e-03, 1.64973408154764161e-03, -2.18115400231975066e-04, 2.25561925434028513e-05, -1.92171064162084224e-06, 1.39417941685833057e-07, -8.81437819454510964e-09, 4.94022751046622183e-10, -2.48736000040125539e-11, 1.13698922364128652e-12, -4.75885969840971219e-14, 1.83810766785130326e-15, -6.68739341771007786e-17, 2.18784717775078739e-18};
+
+// kErf64S: degree 13 in w - 0.35, max weighted error 2.1e-17
+static constexpr double kErf64S[14] = {7.23555060735922462e-01, -3.33667518908424665e-01, -1.08733986486557160e-01, 4.84637334808815490e-01, -6.21153760397772481e-01, 3.29746491323714308e-01, 5.01667673483069509e-01, -1.75106977853493495e+00, 2.85783844743687432e+00, -2.65236212829008755e+00, -6.41369989015191155e-01, 8.88867818303855373e+00, -2.04861033696686299e+01, 2.10918241045758066e+01};
+
+// e^x on |x| <= ln(2)/2, and ln 2 = hi + lo (hi of 32 bits: k hi is exact)
+static constexpr double kLn2Hi = 6.93147180369123816e-01, kLn2Lo = 1.90821492927058770e-10;
+// kExp64: degree 11 in x, max weighted error 2.4e-17
+static constexpr double kExp64[12] = {1.00000000000000000e+00, 1.00000000000000000e+00, 5.00000000000001776e-01, 1.66666666666661467e-01, 4.16666666664930463e-02, 8.33333333356924000e-03, 1.38888889511617889e-03, 1.98412694136199634e-04, 2.48014865772065578e-05, 2.75576384411715744e-06, 2.76322758532418786e-07, 2.49894818233006896e-08};
+

@@ -22,6 +22,22 @@ __device__ __forceinline__ float horner(const float (&c)[N], float x)
     return a;
 }
 
+// The coefficients go through scalar registers where they are used (the asm):
+// left to itself the compiler keeps 29 of them in VGPR pairs around the pair
+// loop and spills (U/J of 30,011 particles 2.4 -> 7.3 ms).
+template <int N>
+__device__ __forceinline__ double horner(const double (&c)[N], double x)
+{
+    double a = c[N - 1];
+#pragma unroll
+    for (int k = N - 2; k >= 0; --k) {
+        double ck = c[k];
+        asm volatile("" : "+s"(ck));
+        a = fma(a, x, ck);
+    }
+    return a;
+}
+
 // Near/far split per source: a source is "near" a wave when some lane has
 // r^2 < q_far^2 sigma^2.  Near sources take the full kernel evaluation and
 // the hi/lo position correction; far sources use the cheap form.
@@ -515,7 +531,8 @@ __device__ __forceinline__ void pair_f64(double tx, double ty, double tz, const 
 //  * Winckelmans (g -> 1 only as 1 - 1.9/q^4) and singular (r = 0 guard):
 //    every pair takes the near form.
 // Near pairs use the reference's g and dg/dq (g_dgdr_ref) at q = r / sigma,
-// except Winckelmans, whose reduced form has no cancellation and no division.
+// except Winckelmans, whose reduced form has no cancellation and no division,
+// and Gaussian-erf (FP64 fits).
 template <int K> struct Far64 { static constexpr double q2 = 0.0; static constexpr bool cheap = false; };
 template <> struct Far64<VPM_KERNEL_GAUSSIANERF> { static constexpr double q2 = 100.0; static constexpr bool cheap = true; };
 template <> struct Far64<VPM_KERNEL_GAUSSIAN> { static constexpr double q2 = 13.0; static constexpr bool cheap = true; };
@@ -623,6 +640,16 @@ __device__ __forceinline__ void accum_pair64(double dx, double dy, double dz, do
     acc[13] = fma(hy, dz, acc[13]);
 }
 
+// e^x for x <= 0: 2^k e^r, |r| <= ln(2)/2 (0 below e^-800; straight-line, and
+// its coefficients stay out of the VGPRs, unlike the library's)
+__device__ __forceinline__ double exp_neg(double x)
+{
+    const double y = fmax(x, -800.0);
+    const double k = rint(y * 1.4426950408889634);
+    const double r = fma(-k, kLn2Lo, fma(-k, kLn2Hi, y));
+    return ldexp(horner(kExp64, r), (int)k);
+}
+
 // a = (x, y, z, far threshold), b = (Gamma' = -Gamma / 4 pi, 1/sigma)
 template <int K>
 __device__ __forceinline__ void near_pair64(double tx, double ty, double tz, const double4 a, const double4 b,
@@ -643,6 +670,35 @@ __device__ __forceinline__ void near_pair64(double tx, double ty, double tz, con
             const double s3 = s2 * b.w;
             accum_pair64(dx, dy, dz, (t + 2.5) * w2s * s3, (t + 3.5) * w2s * w * s3 * s2, b, acc);
         }
+        return;
+    }
+    if constexpr (K == VPM_KERNEL_GAUSSIANERF) {
+        // One exp and two fits (kernel_fits.h) in straight-line code.  custom_erf64
+        // runs every branch that a lane of the wave needs, up to four with two
+        // exps and a division each.  Below q = 2 phi1 and phi0 = t phi1 +
+        // sqrt(2/pi) E/3 have no cancellation; above, as coef_full.
+        // 122 VALU instructions.  U/J of the 12,000 / 30,011 / 100,003 cloud
+        // 525 / 2,418 / 21,250 -> 394 / 1,944 / 18,108 us, of 8,000 ring
+        // particles 394 -> 213, of the 100,003 jet 15,072 -> 14,479; J of a
+        // particle of the 3,001 cloud against 30 digits 2.8e-14 -> 4e-16.
+        const double ri = rsqrt_pos(r2);
+        const double s2 = b.w * b.w;
+        const double t = r2 * s2;                    // q^2
+        const double E = exp_neg(-0.5 * t);
+        const double s3 = s2 * b.w;
+        const double c2E = kConst2 * E;
+        const double p1 = horner(kErf64Phi1, t - kErf64TMid);
+        const double w = ri * (a.w * (b.w * (1.0 / Far64<K>::q2)));   // 1/q: a.w = q2 sigma^2
+        const double q = r2 * ri * b.w;
+        const double g = fma(-E, fma(horner(kErf64S, w - kErf64WMid), w, kConst2 * q), 1.0);
+        const double hm = fma((-1.0 / 3.0) * t, c2E * q, g);          // g - q g'/3
+        const double ri2 = ri * ri;
+        const double ri3 = ri2 * ri;
+        const bool small = t < kErf64TMax;
+        double Fp = small ? fma(t, p1, c2E * (1.0 / 3.0)) * s3 : g * ri3;
+        double Hpp = small ? p1 * (s3 * s2) : hm * (ri3 * ri2);
+        if (!(r2 > 0.0)) { Fp = 0.0; Hpp = 0.0; }    // coincident pairs contribute nothing (fmm.jl:118)
+        accum_pair64(dx, dy, dz, Fp, Hpp, b, acc);
         return;
     }
     if (r2 > 0.0) {   // coincident pairs contribute nothing (fmm.jl:118)
