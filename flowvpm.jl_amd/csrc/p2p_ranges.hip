@@ -7,7 +7,9 @@
 // covering it, in pair order.  A block (or, for FMM leaves, a wave) owns the
 // targets of one item, streams its source ranges through LDS, and adds the
 // result onto its own targets' records: no two blocks write the same
-// particle, and each target's sum runs in pair order.  The pair arithmetic
+// particle, and each target's sum runs in pair order (where several waves share
+// an F32C leaf item, each over its run of ranges, then over the waves in order).
+// The pair arithmetic
 // is p2p_pair.h's.  A plan can be made once and served to U/J, E_str and
 // zeta (vpm_plan_ranges).
 #include <algorithm>
@@ -182,6 +184,68 @@ __global__ __launch_bounds__(kBlock) void ranges_f32c_kernel(const RangeItem* __
     }
 }
 
+// Waves per item of the wave kernels.  A list of few leaves leaves the chip
+// idle with one: 1,001 leaves of 50 particles are one wave per SIMD, which
+// runs its 6,400 sources in a chain of LDS and arithmetic latencies.  Each
+// wave then takes an equal run of the item's source ranges and writes its sums
+// to part[wave][sum][lane], which a finalize kernel adds in order.  Waves of
+// more than 16 targets (R <= 2): up to 32,768 waves, 32 to an item and at
+// least 4 ranges (of 17-64 sources) each; shorter leaves 16,384, 16 and 8.
+// U/J and E_str with one wave per leaf and with this rule: 1,001 leaves of 50
+// 1,777 / 775 -> 513 / 197 us, 79 of 64 417 / 240 -> 96 / 57, 7,408 of 27
+// 1,332 / 470 -> 1,101 / 422, 1,250 of 16 182 / 107 -> 97 / 57 (at 4 ranges a
+// wave 112 / 62), 625 of 8 70 / 45 -> 46 / 31 (55 / 37); 16,384 of 16 keep one
+// (two: 993 / 450 -> 971 / 436).
+static int list_splits(const DevPlan& dp)
+{
+    const bool wide = dp.R <= 2;
+    const int64_t waves = wide ? 32768 : 16384, most = wide ? 32 : 16, ranges = wide ? 4 : 8;
+    return (int)std::max<int64_t>(1, std::min<int64_t>({most, waves / dp.nitems, dp.nsrc / dp.nitems / ranges}));
+}
+
+// The source ranges of the k-th of S waves of an item
+__device__ __forceinline__ void take_split(RangeItem& it, int k, int S)
+{
+    const int64_t b = it.l_begin, n = it.l_end - b;
+    it.l_begin = b + n * k / S;
+    it.l_end = b + n * (k + 1) / S;
+}
+
+template <int NA>
+__device__ __forceinline__ void put_wave(double* __restrict__ part, int64_t w, int lane, const double (&a)[NA])
+{
+    double* o = part + w * NA * 64 + lane;
+#pragma unroll
+    for (int c = 0; c < NA; ++c) o[c * 64] = a[c];
+}
+
+// Sums of target `slot` (lane) of an item over its S waves
+template <int NA>
+__device__ __forceinline__ void sum_waves(const double* __restrict__ part, int64_t item, int S, int slot,
+                                          double (&a)[NA])
+{
+#pragma unroll
+    for (int c = 0; c < NA; ++c) a[c] = 0.0;
+    for (int k = 0; k < S; ++k) {
+        const double* p = part + (item * S + k) * NA * 64 + slot;
+#pragma unroll
+        for (int c = 0; c < NA; ++c) a[c] += p[c * 64];
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void ranges_finalize_kernel(const RangeItem* __restrict__ items, int64_t nitems,
+                                                                 const double* __restrict__ part, int S,
+                                                                 double* __restrict__ P)
+{
+    const int64_t item = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+    if (item >= nitems) return;
+    const int64_t t = items[item].t_begin + (threadIdx.x & 63);
+    if (t >= items[item].t_end) return;
+    double a[kAccF32];
+    sum_waves(part, item, S, threadIdx.x & 63, a);
+    add_f32c_to_record(P + t * NF, a);
+}
+
 // F32C over short target intervals (FMM leaves): each wave owns one item of
 // at most 64 / R targets and stages sources through its own 64-row LDS slot,
 // with no block-wide barrier (within a wave LDS accesses complete in issue
@@ -208,7 +272,8 @@ __global__ __launch_bounds__(kBlock, R > 1 ? 6 : 4) void ranges_wave_f32c_kernel
                                                                   const double* __restrict__ pos, int64_t ld,
                                                                   const float4* __restrict__ gs,
                                                                   const float* __restrict__ cut,
-                                                                  double* __restrict__ P)
+                                                                  double* __restrict__ P, int S,
+                                                                  double* __restrict__ part)
 {
     static_assert(R == 1 || R == 2 || R == 4 || R == 8, "replication");
     constexpr int TW = 64 / R;                  // targets per wave
@@ -220,11 +285,13 @@ __global__ __launch_bounds__(kBlock, R > 1 ? 6 : 4) void ranges_wave_f32c_kernel
     // ranges are read with scalar loads and the stream bookkeeping is SALU)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t w = xcd_block(blockIdx.x, gridDim.x) * (kBlock / 64) + wave;
-    if (w >= nitems) return;   // no block barrier below
+    if (w >= nitems * S) return;   // no block barrier below
     float4* lpos = lpos_all[wave];
     float4* lgs = lgs_all[wave];
     float4* llo = llo_all[wave];
-    const RangeItem it = items[w];
+    const uint32_t wi = S == 1 ? (uint32_t)w : (uint32_t)w / (uint32_t)S;   // fits: RangeItems fit the grid
+    RangeItem it = items[wi];
+    if (S > 1) take_split(it, (int)((uint32_t)w - wi * (uint32_t)S), S);
     const int64_t ib = it.t_begin;
     const double ox = pos[ib], oy = pos[ld + ib], oz = pos[2 * ld + ib];
     const int g = lane / TW;
@@ -274,7 +341,8 @@ __global__ __launch_bounds__(kBlock, R > 1 ? 6 : 4) void ranges_wave_f32c_kernel
             double a[kAccF32];
 #pragma unroll
             for (int c = 0; c < kAccF32; ++c) a[c] = (double)sum[c] + (double)err[c];
-            add_f32c_to_record(P + t * NF, a);
+            if (S == 1) add_f32c_to_record(P + t * NF, a);
+            else put_wave(part, w, lane, a);
         }
         return;
     }
@@ -370,7 +438,10 @@ __global__ __launch_bounds__(kBlock, R > 1 ? 6 : 4) void ranges_wave_f32c_kernel
             for (int c = 0; c < kAccF32; ++c) a[c] += __shfl_xor(a[c], m);
         }
     }
-    if (g == 0 && active) add_f32c_to_record(P + t * NF, a);
+    if (g == 0 && active) {
+        if (S == 1) add_f32c_to_record(P + t * NF, a);
+        else put_wave(part, w, lane, a);
+    }
 }
 
 #pragma clang fp contract(off)
@@ -541,6 +612,7 @@ int make_dev_plan(vpm_field f, const int64_t* tb, const int64_t* te, const int64
     out.items = (const RangeItem*)base;
     out.src = (const int2*)(base + sink.items_bytes());
     out.nitems = shape.nitems;
+    out.nsrc = shape.nsrc;
     out.wave = shape.wave;
     out.R = shape.R;
     return VPM_OK;
@@ -585,9 +657,13 @@ int launch_p2p_plan(vpm_field f, int kernel, int precision, const DevPlan& dp)
         }
     } else if (dp.wave) {
         const int64_t ni = dp.nitems;
-        const dim3 wgrid((unsigned)((ni + kBlock / 64 - 1) / (kBlock / 64)));
+        const int S = list_splits(dp);
+        if (S > 1)
+            if (int rc = ensure(f->part, sizeof(double) * kAccF32 * 64 * (size_t)(ni * S))) return rc;
+        double* part = (double*)f->part.p;
+        const auto blocks = [](int64_t waves) { return dim3((unsigned)((waves + kBlock / 64 - 1) / (kBlock / 64))); };
         switch (kernel) {
-#define VPM_RWR(KID, R) hipLaunchKernelGGL((ranges_wave_f32c_kernel<KID, R>), wgrid, dim3(kBlock), 0, f->stream, d_items, ni, d_src, st.pos, st.ld, st.gs, st.cut, f->P)
+#define VPM_RWR(KID, R) hipLaunchKernelGGL((ranges_wave_f32c_kernel<KID, R>), blocks(ni * S), dim3(kBlock), 0, f->stream, d_items, ni, d_src, st.pos, st.ld, st.gs, st.cut, f->P, S, part)
 #define VPM_RW(KID)                                                                   \
     case KID:                                                                         \
         switch (dp.R) {                                                               \
@@ -602,6 +678,9 @@ int launch_p2p_plan(vpm_field f, int kernel, int precision, const DevPlan& dp)
 #undef VPM_RWR
         default: return fail(VPM_EINVAL, "unknown kernel id");
         }
+        if (S > 1)
+            hipLaunchKernelGGL(ranges_finalize_kernel, blocks(ni), dim3(kBlock), 0, f->stream, d_items, ni,
+                               (const double*)part, S, f->P);
     } else {
         switch (kernel) {
 #define VPM_R32(KID) case KID: hipLaunchKernelGGL(ranges_f32c_kernel<KID>, grid, dim3(kBlock), 0, f->stream, d_items, d_src, st.pos, st.ld, st.gs, st.cut, f->P); break;
@@ -882,12 +961,27 @@ __global__ __launch_bounds__(kBlock) void estr_ranges_f32c_kernel(const RangeIte
 // longer ones; chains of 16 doubled it on 5-particle leaves for 4-8 % less time.
 constexpr int kEstrFold = 4;
 
+// SFS += J'^T A - B of a target (A and B: sums 0-2 and 3-5), J' = J - J_ref
+__device__ __forceinline__ void add_estr_to_record(double* rec, const double (&Jr)[9], int transposed,
+                                                   const double (&A)[6])
+{
+    double Jp[9];
+#pragma unroll
+    for (int c = 0; c < 9; ++c) Jp[c] = rec[RJ + c] - Jr[c];
+    for (int q = 0; q < 3; ++q) {
+        const double S = transposed ? Jp[3 * q] * A[0] + Jp[3 * q + 1] * A[1] + Jp[3 * q + 2] * A[2] - A[3 + q]
+                                    : Jp[q] * A[0] + Jp[3 + q] * A[1] + Jp[6 + q] * A[2] - A[3 + q];
+        rec[RSFS + q] += S;
+    }
+}
+
 template <int K, int R>
 __global__ __launch_bounds__(kBlock) void estr_ranges_wave_f32c_kernel(const RangeItem* __restrict__ items,
                                                                        int64_t nitems,
                                                                        const int2* __restrict__ lsrc,
                                                                        const ListSrc S,
-                                                                       double* __restrict__ P, int transposed)
+                                                                       double* __restrict__ P, int transposed,
+                                                                       int nsplit, double* __restrict__ part)
 {
     static_assert(R == 1 || R == 2 || R == 4 || R == 8, "replication");
     constexpr int TW = 64 / R;
@@ -900,12 +994,14 @@ __global__ __launch_bounds__(kBlock) void estr_ranges_wave_f32c_kernel(const Ran
     // ranges are read with scalar loads and the stream bookkeeping is SALU)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t w = xcd_block(blockIdx.x, gridDim.x) * (kBlock / 64) + wave;
-    if (w >= nitems) return;   // no block barrier below
+    if (w >= nitems * nsplit) return;   // no block barrier below
     float4* lp = lp_all[wave];
     float4* lg = lg_all[wave];
     float4* lq = lq_all[wave];
     float4* ll = ll_all[wave];
-    const RangeItem it = items[w];
+    const uint32_t wi = nsplit == 1 ? (uint32_t)w : (uint32_t)w / (uint32_t)nsplit;
+    RangeItem it = items[wi];
+    if (nsplit > 1) take_split(it, (int)((uint32_t)w - wi * (uint32_t)nsplit), nsplit);
     const double* r0 = P + it.t_begin * NF;
     double Jr[9];
 #pragma unroll
@@ -1086,16 +1182,25 @@ __global__ __launch_bounds__(kBlock) void estr_ranges_wave_f32c_kernel(const Ran
         }
     }
     if (g == 0 && active) {
-        double* rec = P + t * NF;
-        double Jp[9];
-#pragma unroll
-        for (int c = 0; c < 9; ++c) Jp[c] = rec[RJ + c] - Jr[c];
-        for (int q = 0; q < 3; ++q) {
-            const double S = transposed ? Jp[3 * q] * A[0] + Jp[3 * q + 1] * A[1] + Jp[3 * q + 2] * A[2] - A[3 + q]
-                                        : Jp[q] * A[0] + Jp[3 + q] * A[1] + Jp[6 + q] * A[2] - A[3 + q];
-            rec[RSFS + q] += S;
-        }
+        if (nsplit == 1) add_estr_to_record(P + t * NF, Jr, transposed, A);
+        else put_wave(part, w, lane, A);
     }
+}
+
+__global__ __launch_bounds__(kBlock) void estr_ranges_finalize_kernel(const RangeItem* __restrict__ items,
+                                                                      int64_t nitems, const double* __restrict__ part,
+                                                                      int nsplit, double* __restrict__ P,
+                                                                      int transposed)
+{
+    const int64_t item = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+    if (item >= nitems) return;
+    const int64_t t0 = items[item].t_begin, t = t0 + (threadIdx.x & 63);
+    if (t >= items[item].t_end) return;
+    double A[6], Jr[9];
+    sum_waves(part, item, nsplit, threadIdx.x & 63, A);
+#pragma unroll
+    for (int c = 0; c < 9; ++c) Jr[c] = P[t0 * NF + RJ + c];
+    add_estr_to_record(P + t * NF, Jr, transposed, A);
 }
 
 #pragma clang fp contract(off)
@@ -1270,9 +1375,13 @@ int launch_estr_plan(vpm_field f, int kernel, int precision, int transposed, con
     }
     if (!f64 && dp.wave) {
         const int64_t ni = dp.nitems;
-        const dim3 wgrid((unsigned)((ni + kBlock / 64 - 1) / (kBlock / 64)));
+        const int nsplit = list_splits(dp);
+        if (nsplit > 1)
+            if (int rc = ensure(f->part, sizeof(double) * 6 * 64 * (size_t)(ni * nsplit))) return rc;
+        double* part = (double*)f->part.p;
+        const auto blocks = [](int64_t waves) { return dim3((unsigned)((waves + kBlock / 64 - 1) / (kBlock / 64))); };
         switch (kernel) {
-#define VPM_EWR(KID, R) hipLaunchKernelGGL((estr_ranges_wave_f32c_kernel<KID, R>), wgrid, dim3(kBlock), 0, f->stream, d_items, ni, d_src, S, f->P, transposed)
+#define VPM_EWR(KID, R) hipLaunchKernelGGL((estr_ranges_wave_f32c_kernel<KID, R>), blocks(ni * nsplit), dim3(kBlock), 0, f->stream, d_items, ni, d_src, S, f->P, transposed, nsplit, part)
 #define VPM_EW(KID)                                                                   \
     case KID:                                                                         \
         switch (dp.R) {                                                               \
@@ -1287,6 +1396,9 @@ int launch_estr_plan(vpm_field f, int kernel, int precision, int transposed, con
 #undef VPM_EWR
         default: return fail(VPM_EINVAL, "unknown kernel id");
         }
+        if (nsplit > 1)
+            hipLaunchKernelGGL(estr_ranges_finalize_kernel, blocks(ni), dim3(kBlock), 0, f->stream, d_items, ni,
+                               (const double*)part, nsplit, f->P, transposed);
     } else if (f64) {
         switch (kernel) {
 #define VPM_EG64(KID, G)                                                                                        \

@@ -110,7 +110,7 @@ namespace vpm {
 struct DevPlan {
     const RangeItem* items = nullptr;
     const int2* src = nullptr;
-    int64_t nitems = 0;
+    int64_t nitems = 0, nsrc = 0;
     bool wave = false;   // F32C wave kernels (FMM leaves)
     int R = 1;           // lane groups per target of the wave kernels
 };
