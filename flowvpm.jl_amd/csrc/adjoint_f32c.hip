@@ -268,14 +268,14 @@ __device__ __forceinline__ void adj_group(const AdjTarget& T, const float4* pa, 
     }
 }
 
-// partT [nss][3][np]: target-side sums per source super-tile.
-// partS [ntt][7][np]: source-side sums per target super-tile.
+// partT [nss nph][3][np]: target-side sums per source super-tile and part.
+// partS [ntt nph][7][np]: source-side sums per target super-tile and part.
 // tcot [4][np] float4: (Ubar, tau_x), (Jbar col 0, tau_y), (col 1, tau_z), (col 2, 0).
 // JB = false: every Jbar is zero, and only tcot[0] is read.
 template <int K, bool JB>
 __global__ __launch_bounds__(kBlock) void adj_f32c_kernel(
     const double* __restrict__ pos, int64_t ld, const float4* __restrict__ sgs, const float* __restrict__ scut,
-    const float4* __restrict__ tcot, int64_t np, int64_t tsz, int64_t ssz, int ntt, int nss, int remap,
+    const float4* __restrict__ tcot, int64_t np, int64_t tsz, int64_t ssz, int ntt, int nss, int nph, int remap,
     double* __restrict__ partT, double* __restrict__ partS)
 {
     __shared__ float4 lpos[kAdjGroups][128];   // s'_hi, far-field r^2 threshold
@@ -292,8 +292,12 @@ __global__ __launch_bounds__(kBlock) void adj_f32c_kernel(
     // they re-read in that XCD's L2.
     int64_t L = blockIdx.x;
     if (remap) L = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    const int part = (int)(L % nph);   // the block's phases, of nph equal parts
+    L /= nph;
     const int tt = (int)(L / nss);
     const int ss = (int)(L % nss);
+    const int64_t rowT = (int64_t)ss * nph + part, rowS = (int64_t)tt * nph + part;
+    const int ph0 = part * kAdjGroups / nph, ph1 = (part + 1) * kAdjGroups / nph;
     const int64_t tb = (int64_t)tt * tsz, te = min(tb + tsz, np);
     const int64_t sb = (int64_t)ss * ssz, se = min(sb + ssz, np);
 
@@ -357,12 +361,12 @@ __global__ __launch_bounds__(kBlock) void adj_f32c_kernel(
             double prev[3] = {0.0, 0.0, 0.0};
             if (tvalid && !first) {
 #pragma unroll
-                for (int c = 0; c < 3; ++c) prev[c] = partT[((int64_t)ss * 3 + c) * np + i];
+                for (int c = 0; c < 3; ++c) prev[c] = partT[(rowT * 3 + c) * np + i];
             }
             const WaveBox tbx = wave_box(T.x, T.y, T.z);
             const bool wactive = tc + wave * 64 < te;
             float X[3] = {0.f, 0.f, 0.f};
-            for (int ph = 0; ph < kAdjGroups; ++ph) {
+            for (int ph = ph0; ph < ph1; ++ph) {
                 const int g = (wave + ph) & (kAdjGroups - 1);
                 if (wactive && g * 64 < nv) {
                     const float* gb = lbox[g];
@@ -387,12 +391,12 @@ __global__ __launch_bounds__(kBlock) void adj_f32c_kernel(
             }
             if (tvalid) {
 #pragma unroll
-                for (int c = 0; c < 3; ++c) partT[((int64_t)ss * 3 + c) * np + i] = prev[c] + (double)X[c];
+                for (int c = 0; c < 3; ++c) partT[(rowT * 3 + c) * np + i] = prev[c] + (double)X[c];
             }
         }
         if (tid < nv) {
 #pragma unroll
-            for (int c = 0; c < kAdjAcc; ++c) partS[((int64_t)tt * kAdjAcc + c) * np + sc + tid] = lacc[c][tid];
+            for (int c = 0; c < kAdjAcc; ++c) partS[(rowS * kAdjAcc + c) * np + sc + tid] = lacc[c][tid];
         }
     }
 }
@@ -415,36 +419,47 @@ __global__ __launch_bounds__(kBlock) void pack_adj_cot_kernel(const double* __re
     tcot[3 * np + k] = make_float4((float)J[6], (float)J[7], (float)J[8], 0.f);
 }
 
-// Sums the super-tile partials in fixed order and scatters to particle order.
+// Sums the super-tile partials in fixed order and scatters to particle order:
+// a block serves kSumSet particles with kSumParts threads each, as sum_splits
+// (with one thread per particle, N = 32,768 was 128 blocks and a chain of 832
+// loads each: adjoint 2,815 -> 2,775 us).
 __global__ __launch_bounds__(kBlock) void adj_finalize_kernel(const double* __restrict__ partT, int nss,
                                                               const double* __restrict__ partS, int ntt, int64_t np,
                                                               const uint32_t* __restrict__ perm,
                                                               double* __restrict__ Xbar, double* __restrict__ Gbar,
                                                               double* __restrict__ Sbar)
 {
-    const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (k >= np) return;
-    double x[3] = {0.0, 0.0, 0.0}, g[3] = {0.0, 0.0, 0.0}, s = 0.0;
-    for (int b = 0; b < nss; ++b) {
+    __shared__ double red[kSumParts - 1][kAdjAcc][kSumSet];
+    const int t = threadIdx.x & (kSumSet - 1), r = threadIdx.x / kSumSet;
+    const int64_t k = (int64_t)blockIdx.x * kSumSet + t;
+    double a[kAdjAcc] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};   // dX, dGamma', dsigma
+    if (k < np) {
+        for (int b = r; b < nss; b += kSumParts) {
 #pragma unroll
-        for (int c = 0; c < 3; ++c) x[c] += partT[((int64_t)b * 3 + c) * np + k];
-    }
-    for (int b = 0; b < ntt; ++b) {
-        const double* ps = partS + (int64_t)b * kAdjAcc * np + k;
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            x[c] += ps[c * np];
-            g[c] += ps[(3 + c) * np];
+            for (int c = 0; c < 3; ++c) a[c] += partT[((int64_t)b * 3 + c) * np + k];
         }
-        s += ps[6 * np];
+        for (int b = r; b < ntt; b += kSumParts) {
+#pragma unroll
+            for (int c = 0; c < kAdjAcc; ++c) a[c] += partS[((int64_t)b * kAdjAcc + c) * np + k];
+        }
     }
+    if (r > 0) {
+#pragma unroll
+        for (int c = 0; c < kAdjAcc; ++c) red[r - 1][c][t] = a[c];
+    }
+    __syncthreads();
+    if (r > 0 || k >= np) return;
+#pragma unroll
+    for (int q = 0; q < kSumParts - 1; ++q)
+#pragma unroll
+        for (int c = 0; c < kAdjAcc; ++c) a[c] += red[q][c][t];
     const int64_t p = perm ? (int64_t)perm[k] : k;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-        Xbar[3 * p + c] = x[c];
-        Gbar[3 * p + c] = -kConst4 * g[c];
+        Xbar[3 * p + c] = a[c];
+        Gbar[3 * p + c] = -kConst4 * a[3 + c];
     }
-    Sbar[p] = s;
+    Sbar[p] = a[6];
 }
 
 // Super-tiles, each a whole number of 256-particle chunks: up to 64 on the
@@ -468,6 +483,12 @@ static void adj_tiles(int64_t np, int64_t& tsz, int& ntt, int64_t& ssz, int& nss
     nss = (int)((np + ssz - 1) / ssz);
 }
 
+// Most super-tile pairs of a launch that gives each of their four phases a block
+// of its own.  Adjoint (U and J) of 200 / 1,000 / 3,001 / 5,000 / 8,000
+// particles, with transfers: 221 / 242 / 237 / 276 / 411 -> 140 / 154 / 173 /
+// 221 / 364 us; from 1,024 pairs up the chip is full and the staging repeats.
+constexpr int64_t kAdjPartBlocks = 1024;
+
 int launch_uj_adjoint_f32c(vpm_field f, int kernel, const double* dU, const double* dJ, double* dX, double* dG,
                            double* dS, float4* tcot, bool jbar)
 {
@@ -484,11 +505,13 @@ int launch_uj_adjoint_f32c(vpm_field f, int kernel, const double* dU, const doub
     int64_t tsz, ssz;
     int ntt, nss;
     adj_tiles(np, tsz, ntt, ssz, nss);
-    const size_t nT = (size_t)nss * 3 * (size_t)np, nS = (size_t)ntt * kAdjAcc * (size_t)np;
+    // each phase to a block of its own where the super-tiles leave the chip idle
+    const int nph = (int64_t)ntt * nss <= kAdjPartBlocks ? kAdjGroups : 1;
+    const size_t nT = (size_t)nss * nph * 3 * (size_t)np, nS = (size_t)ntt * nph * kAdjAcc * (size_t)np;
     if ((rc = ensure(f->part, sizeof(double) * (nT + nS)))) return rc;
     double* partT = (double*)f->part.p;
     double* partS = partT + nT;
-    const unsigned grid = (unsigned)ntt * (unsigned)nss;
+    const unsigned grid = (unsigned)ntt * (unsigned)nss * (unsigned)nph;
     const int remap = (grid % 8 == 0) ? 1 : 0;
     timing_begin(f);
     switch (kernel) {
@@ -496,11 +519,11 @@ int launch_uj_adjoint_f32c(vpm_field f, int kernel, const double* dU, const doub
     case KID:                                                                                                 \
         if (jbar)                                                                                             \
             hipLaunchKernelGGL((adj_f32c_kernel<KID, true>), dim3(grid), dim3(kBlock), 0, f->stream, S.pos,     \
-                               S.ld, S.gs, S.cut, (const float4*)tcot, np, tsz, ssz, ntt, nss, remap, partT,  \
+                               S.ld, S.gs, S.cut, (const float4*)tcot, np, tsz, ssz, ntt, nss, nph, remap, partT,  \
                                partS);                                                                        \
         else                                                                                                  \
             hipLaunchKernelGGL((adj_f32c_kernel<KID, false>), dim3(grid), dim3(kBlock), 0, f->stream, S.pos,    \
-                               S.ld, S.gs, S.cut, (const float4*)tcot, np, tsz, ssz, ntt, nss, remap, partT,  \
+                               S.ld, S.gs, S.cut, (const float4*)tcot, np, tsz, ssz, ntt, nss, nph, remap, partT,  \
                                partS);                                                                        \
         break;
         VPM_ADJ32(VPM_KERNEL_SINGULAR)
@@ -514,8 +537,8 @@ int launch_uj_adjoint_f32c(vpm_field f, int kernel, const double* dU, const doub
     e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "adj_f32c");
     timing_end(f, 3);
-    hipLaunchKernelGGL(adj_finalize_kernel, dim3(nb), dim3(kBlock), 0, f->stream, partT, nss, partS, ntt, np, S.perm,
-                       dX, dG, dS);
+    hipLaunchKernelGGL(adj_finalize_kernel, dim3(sum_blocks(np)), dim3(kBlock), 0, f->stream, partT, nss * nph, partS,
+                       ntt * nph, np, S.perm, dX, dG, dS);
     e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "adj_finalize");
     return VPM_OK;
