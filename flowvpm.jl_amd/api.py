@@ -164,6 +164,7 @@ class Field:
 
     def get_particles(self, out, rows=(0, NFIELDS), np_=None):
         assert out.dtype == np.float64 and out.flags.c_contiguous and out.shape[1] == NFIELDS
+        _check_writeable(out)
         n = out.shape[0] if np_ is None else np_
         check(lib().vpm_get_particles(self.handle, out.ctypes.data_as(_lib._dptr), n, rows[0], rows[1]))
         return out
@@ -425,6 +426,20 @@ def _as_matrix(target):
     return P
 
 
+def _check_writeable(P):
+    """The library writes through the array's address, past numpy's own check."""
+    if not P.flags.writeable:
+        raise ValueError("particle array is read-only")
+
+
+def _as_target(target):
+    """_as_matrix of particles that the call writes to, refused before any work."""
+    P = _as_matrix(target)
+    if P.shape[0]:
+        _check_writeable(P)
+    return P
+
+
 # ---------------------------------------------------------------- UJ functors
 def UJ_hip(pfield, *, reset=True, reset_sfs=False, sfs=False, kernel=None, precision=None,
            transposed=None, device=None, sort=True, rbf=False):
@@ -432,7 +447,7 @@ def UJ_hip(pfield, *, reset=True, reset_sfs=False, sfs=False, kernel=None, preci
     on the GPU.  Accepts a ParticleField or an (n, 46) record matrix; mutates
     U, vorticity, J, PSE (reset) and SFS rows in place.  `rbf` is ignored, as
     in the reference."""
-    P = _as_matrix(pfield)
+    P = _as_target(pfield)
     pf = pfield if isinstance(pfield, ParticleField) else None
     kernel = kernel or (pf.kernel if pf else kernel_default)
     precision = precision or (pf.precision if pf else "f32c")
@@ -457,7 +472,7 @@ def _copy_back(f, P, with_sfs):
 def UJ_hip_fields(source, target, *, kernel=None, precision=None, device=None):
     """UJ_direct(source, target) (FLOWVPM_UJ.jl:48-50): accumulates the
     influence of every particle of `source` on every particle of `target`."""
-    S, T = _as_matrix(source), _as_matrix(target)
+    S, T = _as_matrix(source), _as_target(target)
     kernel = kernel or (source.kernel if isinstance(source, ParticleField) else kernel_default)
     precision = precision or (source.precision if isinstance(source, ParticleField) else "f32c")
     device = device if device is not None else 0
@@ -476,7 +491,7 @@ def UJ_hip_fields(source, target, *, kernel=None, precision=None, device=None):
 def p2p_ranges(pfield, tb, te, sb, se, *, kernel=None, precision=None, device=None):
     """fmm.direct! over a batch of 0-based half-open (target, source) range
     pairs of one field (FLOWVPM_fmm.jl:102-168); accumulates U and J."""
-    P = _as_matrix(pfield)
+    P = _as_target(pfield)
     kernel = kernel or (pfield.kernel if isinstance(pfield, ParticleField) else kernel_default)
     precision = precision or (pfield.precision if isinstance(pfield, ParticleField) else "f32c")
     f = _scratch_field(P.shape[0], 0 if device is None else device)
@@ -494,7 +509,7 @@ def estr_ranges(pfield, tb, te, sb, se, *, kernel=None, precision=None, transpos
     """Estr_fmm! over a direct list of 0-based half-open (target, source)
     range pairs (FLOWVPM_subfilterscale_models.jl:157-188): E_str pairs onto
     SFS, no static skip, no reset."""
-    P = _as_matrix(pfield)
+    P = _as_target(pfield)
     pf = pfield if isinstance(pfield, ParticleField) else None
     kernel = kernel or (pf.kernel if pf else kernel_default)
     precision = precision or (pf.precision if pf else "f32c")
@@ -514,7 +529,7 @@ def zeta_ranges(pfield, tb, te, sb, se, *, kernel=None, precision=None, device=N
     """zeta_fmm's pair loop (FLOWVPM_viscous.jl:523-558) over a direct list
     of 0-based half-open (target, source) range pairs: J[1:3] += the zeta
     field of the sources, no reset, no static skip."""
-    P = _as_matrix(pfield)
+    P = _as_target(pfield)
     pf = pfield if isinstance(pfield, ParticleField) else None
     kernel = kernel or (pf.kernel if pf else kernel_default)
     precision = precision or (pf.precision if pf else "f32c")
@@ -531,7 +546,7 @@ def zeta_ranges(pfield, tb, te, sb, se, *, kernel=None, precision=None, device=N
 
 def Estr_hip(pfield, *, kernel=None, precision=None, transposed=None, device=None):
     """Estr_direct! (FLOWVPM_subfilterscale_models.jl:43-92) on the GPU."""
-    P = _as_matrix(pfield)
+    P = _as_target(pfield)
     pf = pfield if isinstance(pfield, ParticleField) else None
     kernel = kernel or (pf.kernel if pf else kernel_default)
     precision = precision or (pf.precision if pf else "f32c")
