@@ -100,7 +100,10 @@ struct Ring {
     }
 };
 
-// Events of the pieces in flight, for one call.
+// Events of the pieces in flight, for one call.  With a release to the system:
+// the gather kernel writes pinned pieces that need not be coherent, and the
+// host reads one after its event, with later pieces still in flight (no wait
+// for the stream between).
 struct Events {
     hipEvent_t ev[kSlots] = {};
     ~Events()
@@ -111,7 +114,7 @@ struct Events {
     int make(int n)
     {
         for (int s = 0; s < n; ++s) {
-            const hipError_t e = hipEventCreateWithFlags(&ev[s], hipEventDisableTiming);
+            const hipError_t e = hipEventCreateWithFlags(&ev[s], hipEventDisableTiming | hipEventReleaseToSystem);
             if (e != hipSuccess) return hip_fail(e, "hipEventCreate");
         }
         return VPM_OK;
