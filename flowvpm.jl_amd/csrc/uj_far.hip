@@ -15,34 +15,41 @@
 // pair; here the VALU only turns r^2 into H (rsq, two products, and the two
 // FP16 halves), and the matrix cores do both contractions.
 //
-//  * r^2 of 32 sources x 32 targets is one 32x32x16 product: 16 terms
-//    -2 s.t + s^2 + t^2 with s and t split into two FP16 parts each.
-//  * H = h1 + h2 and column = c1 + c2 in FP16 parts (22 bits or more, as
-//    FP32 products round), h1 c1 + h1 c2 + h2 c1 in FP32 accumulators: three
-//    32x32x16 products per 16 sources.  The r^2 product leaves a lane with
-//    its target's H in exactly the register order the second product reads
-//    as its left operand (the sources in permuted order, which the columns'
-//    rows follow), so nothing moves between lanes.
+//  * r^2 of 32 sources x 32 targets is one 32x32x16 product of -2 s.t and t^2,
+//    with s, t and t^2 split into two FP16 parts each, onto s^2 in FP32 as the
+//    accumulator's start: the unit cuts each of 8 products at 2^-24 of the
+//    largest, and s^2 among them would cut the others always toward r^2 = s^2.
+//  * H = h1 + h2 and column = c1 + c2 in FP16 parts (22 bits, of H below 1/4
+//    down to 20, where h2 is subnormal), h1 c1 + h1 c2 + h2 c1 in FP32
+//    accumulators: three 32x32x16 products per 16 sources.  The r^2 product
+//    leaves a lane with its target's H in exactly the register order the
+//    second product reads as its left operand (the sources in permuted order,
+//    which the columns' rows follow), so nothing moves between lanes.
 //  * Scales: positions are divided by R = 2^k >= every |s| and |t| of the
 //    (target block, 256-source tile), strengths by the tile's largest
 //    component (a power of two).  A wave of 64 targets takes a group of 64
 //    sources here when the gap between their boxes is at least the group's
-//    far radius, the wave's reach from the origin (then |s| <= 2 r and the
-//    expansion of r^2 loses at most two bits), and R / 8 (then H <= 2^15 fits
-//    FP16 and H >= 1/32 keeps its second half).  The rest goes to
-//    uj_rest_kernel, the VALU pair code: the bits of one word per (block,
-//    tile), computed once, tell both kernels who takes which group.
-//  * The FP32 accumulators are added to FP64 sums after every tile; the
+//    far radius, the wave's reach from the origin (then |t| <= r, |s| <= 2 r:
+//    the terms of r^2 reach 9 r^2, three bits, those of U 27 r^3, five), and
+//    R / 8 (then H <= 2^15 fits FP16, and r <= 2 R keeps H >= 1/32).  The rest
+//    goes to uj_rest_kernel, the VALU pair code: the bits of one word per
+//    (block, tile), computed once, tell both kernels who takes which group.
+//  * The FP32 accumulators are added to FP64 sums after every 128 sources; the
 //    polynomials in t are formed once per target in FP64.
-// Measured: U/J of the 2^20 jet 702 -> 345 ms (1.57e12 -> 3.2e12 pairs/s), of
-// the 65,536 cloud 3.84 -> 2.60 ms and of the leapfrog rings 3.41 -> 1.92 ms;
-// error against 64 bits of U unchanged (1.6e-7 on the cloud), of J 4.5e-7 ->
-// 3.0e-7 (rest kernel).  The far kernel is bound by the VALU: per pair one
-// rsq (8.3 cycles per wave), three products (2.6 each), two packed conversions
-// of two (4.6) and a fma_mix (4.4) are 25-32 cycles per 64 pairs; the matrix
-// products (7 per 1,024 pairs, 15 cycles per 64) run beside them (two of the
-// three left out changes nothing).  It runs at 44: the clock falls from 2.35
-// to 1.93 GHz under both, and staging and folding add 11 %.
+//  * What is the same for every source does not average out: v_rsq_f32's mean
+//    error (kRsqMean) and the target's rounding (move_u) are taken out of the
+//    sums.
+// Error against 64 bits per unit of the summation scale (RMS over targets), all
+// pairs in FP32 -> here: U of the 2^20 jet 1.3e-8 -> 5.4e-9, of the 65,536
+// leapfrog rings 1.65e-8 -> 1.1e-8 and cloud 1.88e-9 -> 1.86e-9, J 3.8e-8 ->
+// 1.6e-8, 7.7e-8 -> 3.0e-8 and 8.2e-9 -> 5.5e-9 (the rest kernel's shorter
+// chains).  With s^2 among the products, a fold per 256 sources and both means
+// left in, U was 2.4e-8, 1.7e-8 and 1.9e-9, and the jet took 337 ms instead of
+// 353 (s^2 from LDS 8 ms, the second fold 9).
+// Measured: U/J of the 2^20 jet 709 -> 353 ms (1.55e12 -> 3.1e12 pairs/s), of
+// the 65,536 cloud 3.72 -> 2.50 ms and of the leapfrog rings 3.26 -> 1.80 ms.
+// The far kernel is bound by the VALU: per pair one rsq, three products, two
+// packed conversions of two and a fma_mix.
 #include <algorithm>
 #include <cfloat>
 
@@ -59,7 +66,10 @@ constexpr int kCols = 27;            // columns of a source
 constexpr int kColLd = kTile + 8;    // halves per column row in LDS: 33 x 16 bytes, so 16 rows cover all banks
 constexpr int kColShift = 13;        // columns are scaled by 2^13
 constexpr float kLowScale = 64.f;    // scale of the low FP16 part of a position
-constexpr float kSqScale = 4096.f;   // scale of s^2 and t^2 in the r^2 product
+constexpr float kSqScale = 4096.f;   // scale of t^2 in the r^2 product
+// v_rsq_f32 is low by 5.8e-9 of its result on [1, 2) and 8.1e-9 on [2, 4)
+// (means weighted by 1/x), so r^-5 by 3.5e-8 wherever r lies.
+constexpr double kRsqMean = 1.0 + 3.5e-8;
 // The far kernel pays from about 16,384 particles (U/J of the cloud, the jet
 // and the leapfrog rings, with and without it: 0.279 / 0.287, 0.255 / 0.264 and
 // 0.271 / 0.313 ms at 16,384; 0.139 / 0.110 ms for the cloud at 8,192, where
@@ -176,10 +186,15 @@ __global__ __launch_bounds__(kBlock) void far_word_kernel(const double* __restri
     words[(int64_t)blockIdx.x * ntile + tile] = bits | ((uint32_t)(k + 64) & 255u) << 16 | (uint32_t)(ge + 128) << 24;
 }
 
-__device__ __forceinline__ void split16(float x, _Float16& h, _Float16& l)
+__device__ __forceinline__ void split16(double x, _Float16& h, _Float16& l)
 {
-    h = (_Float16)x;
-    l = (_Float16)(x - (float)h);
+    h = (_Float16)(float)x;
+    l = (_Float16)(float)(x - (double)(float)h);
+}
+
+__device__ __forceinline__ double square3(const float (&x)[3])
+{
+    return fma((double)x[2], (double)x[2], fma((double)x[1], (double)x[1], (double)x[0] * x[0]));
 }
 
 // x = h + l / kLowScale; returns the represented value
@@ -193,6 +208,17 @@ __device__ __forceinline__ float split_pos(float x, _Float16& h, _Float16& l)
 __device__ __forceinline__ floatx16 mfma16(half8 a, half8 b, floatx16 c)
 {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+// U of the 14 sums moved by d, to first order (J as in add_f32c_to_record).
+__device__ __forceinline__ void move_u(const double (&d)[3], double (&a)[kAccF32])
+{
+    const double u0 = -3.0 * (a[6] * d[0] + a[9] * d[1] + a[12] * d[2]) + a[5] * d[1] - a[4] * d[2];
+    const double u1 = -3.0 * (a[7] * d[0] + a[10] * d[1] + a[13] * d[2]) - a[5] * d[0] + a[3] * d[2];
+    const double u2 = -3.0 * (a[8] * d[0] + a[11] * d[1] - (a[6] + a[10]) * d[2]) + a[4] * d[0] - a[3] * d[1];
+    a[0] += u0;
+    a[1] += u1;
+    a[2] += u2;
 }
 
 // The 14 sums of accum_pair from the 27 basis sums S of a target at t.
@@ -262,15 +288,16 @@ __global__ __launch_bounds__(kFarThreads, 4) void uj_far_kernel(
     const double* __restrict__ spos, int64_t sld, const float4* __restrict__ sgs, int64_t ns,
     const uint32_t* __restrict__ words, int64_t ntile, int64_t chunk, double* __restrict__ part, int64_t pld)
 {
-    // columns [part][column][source] and the sources' halves of the r^2
-    // product; the basis sums at the end reuse the space, four waves at a time
+    // columns [part][column][source], the sources' halves of the r^2 product
+    // and their s^2; the basis sums at the end reuse the space, four waves at a time
     constexpr int kColBytes = 2 * kCols * kColLd * 2;
     constexpr int kSumLd = kCols + 1;
     constexpr int kSumBytes = 4 * 32 * kSumLd * 8;
-    constexpr int kStageBytes = kColBytes + 2 * kTile * 16;
+    constexpr int kStageBytes = kColBytes + 2 * kTile * 16 + kTile * 4;
     __shared__ __attribute__((aligned(16))) char smem[kStageBytes > kSumBytes ? kStageBytes : kSumBytes];
     _Float16* lcol = (_Float16*)smem;
     half8* lr = (half8*)(smem + kColBytes);
+    float* ls2 = (float*)(smem + kColBytes + 2 * kTile * 16);
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -297,6 +324,7 @@ __global__ __launch_bounds__(kFarThreads, 4) void uj_far_kernel(
 #pragma unroll
     for (int i = 0; i < 16; ++i) sum[i] = 0.0;
     half8 T;
+    float trep[3] = {0.f, 0.f, 0.f};   // the target as T has it (the same in every scale)
     int kcur = 1000;
 
     const int64_t c0 = (int64_t)blockIdx.y * chunk, c1 = min(c0 + chunk, ntile);
@@ -340,11 +368,9 @@ __global__ __launch_bounds__(kFarThreads, 4) void uj_far_kernel(
                     r1[a] = (_Float16)((float)h * (1.f / kLowScale));
                     r1[3 + a] = l;
                 }
-                _Float16 q1, q2;
-                split16(fmaf(st[2], st[2], fmaf(st[1], st[1], st[0] * st[0])) * kSqScale, q1, q2);
-                r0[6] = q1;
-                r0[7] = q2;
-                r1[6] = r1[7] = (_Float16)(1.f / kSqScale);
+                r0[6] = r0[7] = (_Float16)(1.f / kSqScale);
+                r1[6] = r1[7] = (_Float16)0.f;
+                ls2[src] = (float)square3(st);
                 lr[src] = r0;
                 lr[kTile + src] = r1;
                 put(0, g[0], 1, g[1]);
@@ -381,16 +407,33 @@ __global__ __launch_bounds__(kFarThreads, 4) void uj_far_kernel(
                 T[a] = (_Float16)x;
                 T[3 + a] = (_Float16)(x * (hh ? 1.f / (kLowScale * kLowScale) : 1.f / kLowScale));
             }
+            for (int a = 0; a < 3; ++a) trep[a] = ldexpf(st[a], k);
             _Float16 q1, q2;
-            split16(fmaf(st[2], st[2], fmaf(st[1], st[1], st[0] * st[0])) * kSqScale, q1, q2);
-            T[6] = hh ? q1 : (_Float16)(1.f / kSqScale);
-            T[7] = hh ? q2 : (_Float16)(1.f / kSqScale);
+            split16(square3(st) * kSqScale, q1, q2);
+            T[6] = hh ? (_Float16)0.f : q1;
+            T[7] = hh ? (_Float16)0.f : q2;
         }
+        const double sc = ldexp(kRsqMean, ge - kColShift + k * (deg - 5));
+        const auto fold = [&]() {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sum[i] = fma((double)acc[i], sc, sum[i]);
+            acc = zero;
+        };
         for (int g = 0; g < 4; ++g) {
+            if (g == 2) fold();
             if (!((my >> g) & 1u) || tile * kTile + g * 64 >= ns) continue;
             const half8* rp = lr + hh * kTile + g * 64 + m;
             const _Float16* cp = lcol + n * kColLd + g * 64 + hh * 8;
-            const floatx16 ra = mfma16(rp[0], T, zero), rb = mfma16(rp[32], T, zero);
+            floatx16 ra, rb;   // s^2 of the lane's rows, then r^2
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float* p2 = ls2 + g * 64 + 8 * q + 4 * hh;
+                const float4 x = *(const float4*)p2, y = *(const float4*)(p2 + 32);
+                ra[4 * q] = x.x; ra[4 * q + 1] = x.y; ra[4 * q + 2] = x.z; ra[4 * q + 3] = x.w;
+                rb[4 * q] = y.x; rb[4 * q + 1] = y.y; rb[4 * q + 2] = y.z; rb[4 * q + 3] = y.w;
+            }
+            ra = mfma16(rp[0], T, ra);
+            rb = mfma16(rp[32], T, rb);
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
                 const floatx16& r2 = ks < 2 ? ra : rb;
@@ -405,10 +448,7 @@ __global__ __launch_bounds__(kFarThreads, 4) void uj_far_kernel(
                 acc = mfma16(h1, b1, acc);
             }
         }
-        const double sc = ldexp(1.0, ge - kColShift + k * (deg - 5));
-#pragma unroll
-        for (int i = 0; i < 16; ++i) sum[i] = fma((double)acc[i], sc, sum[i]);
-        acc = zero;
+        fold();
     }
     // the wave's 32 targets x 27 sums to LDS, then a target per lane
     for (int half = 0; half < 2; ++half) {
@@ -424,9 +464,16 @@ __global__ __launch_bounds__(kFarThreads, 4) void uj_far_kernel(
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         const int64_t i = i0 + lane;
         if (lane < 32 && i < nt) {
-            double t[3], out[kAccF32];
-            for (int a = 0; a < 3; ++a) t[a] = tpos[a * tld + t0 + i] - O[a];
+            // sums for the target as the weights had it, then moved to its
+            // place: its rounding is the same for every source, and left in
+            // the weights it is the largest error of U
+            double t[3], d[3], out[kAccF32];
+            for (int a = 0; a < 3; ++a) {
+                t[a] = trep[a];
+                d[a] = tpos[a * tld + t0 + i] - O[a] - t[a];
+            }
             far_combine(t, ls + lane * kSumLd, out);
+            move_u(d, out);
             double* o = part + (int64_t)blockIdx.y * kAccF32 * pld + i;
 #pragma unroll
             for (int c = 0; c < kAccF32; ++c) o[c * pld] = out[c];
