@@ -160,8 +160,9 @@ __global__ __launch_bounds__(kBlock) void far_word_kernel(const double* __restri
     int k = 0, ge = 0;
     (void)frexp(sqrt(r2) * (1.0 + 1e-6), &k);   // 2^k > every |s|, |t|
     if (gm > 0.0) (void)frexp(gm * (1.0 + 1e-6), &ge);
-    // scales and their products stay well inside FP32
-    const bool ok = k >= -24 && k <= 24 && ge >= -100 && ge <= 60 && ge - 5 * k <= 100;
+    // scales and their products stay well inside FP32 (frexp gives an
+    // infinity, a strength beyond FP32 or a distance squared, the exponent 0)
+    const bool ok = r2 < INFINITY && gm < INFINITY && k >= -24 && k <= 24 && ge >= -100 && ge <= 60 && ge - 5 * k <= 100;
     const double rmin2 = ldexp(1.0, 2 * k - 6) * (1.0 + 1e-4);
     uint32_t bits = 0;
     for (int w = 0; w < 4; ++w) {
