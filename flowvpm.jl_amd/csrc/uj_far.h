@@ -11,9 +11,6 @@ struct FarSplit {
     int64_t rest = 1;             // rest kernel: splits (every rest-th tile)
 };
 
-// Fewest particles of a field whose time steps take the far kernel.
-constexpr int64_t kFarStepMin = 1 << 16;
-
 // Whether an all-pairs launch is split at all.
 bool far_applies(int kernel, int precision, int64_t nt, int64_t ns);
 // Targets per launch: the words of one launch stay within 256 MiB.
