@@ -26,6 +26,7 @@ int fail(int status, const std::string& msg)
 
 int hip_fail(hipError_t e, const char* what)
 {
+    (void)hipGetLastError();   // reported here: the next launch check is to find its own
     g_last_error = std::string(what) + ": " + hipGetErrorString(e);
     return e == hipErrorOutOfMemory ? VPM_ENOMEM : VPM_EDEVICE;
 }
