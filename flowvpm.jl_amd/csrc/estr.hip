@@ -584,10 +584,13 @@ int launch_estr_impl(vpm_field f, int kernel, int transposed, int precision, con
         // 4,096 blocks of equal work (16 waves per SIMD)
         const int64_t grain = split_grain(nblk(np), np);
         const int64_t steps = (np + grain - 1) / grain;
-        int64_t K = std::min<int64_t>(std::max<int64_t>(1, 4096 / nblk(np)), steps);
-        const int64_t chunk = ((steps + K - 1) / K) * grain;
+        int64_t K = std::min<int64_t>(std::max<int64_t>(1, 4096 / nblk(np)), steps), chunk = 0;
+        rc = fit_splits(K, [&](int64_t m) {
+            chunk = ((steps + m - 1) / m) * grain;
+            return ensure(f->part, sizeof(double) * 3 * (size_t)((np + chunk - 1) / chunk) * (size_t)np);
+        });
+        if (rc) return rc;
         K = (np + chunk - 1) / chunk;
-        if ((rc = ensure(f->part, sizeof(double) * 3 * (size_t)K * (size_t)np))) return rc;
         double* part = (double*)f->part.p;
         const dim3 grid(nblk(np), (unsigned)K);
         timing_begin(f);
@@ -685,8 +688,9 @@ int launch_estr_f64far(vpm_field f, int kernel, int transposed)
                        (const float*)cutf, np, tbox);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "pack_estr64");
-    const int64_t K = near_splits(np);
-    if ((rc = ensure(f->part, sizeof(double) * 3 * (size_t)K * (size_t)np))) return rc;
+    int64_t K = near_splits(np);
+    if ((rc = fit_splits(K, [&](int64_t m) { return ensure(f->part, sizeof(double) * 3 * (size_t)m * (size_t)np); })))
+        return rc;
     double* part = (double*)f->part.p;
     timing_begin(f);
     switch (kernel) {

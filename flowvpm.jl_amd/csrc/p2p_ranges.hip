@@ -203,6 +203,17 @@ static int list_splits(const DevPlan& dp)
     return (int)std::max<int64_t>(1, std::min<int64_t>({most, waves / dp.nitems, dp.nsrc / dp.nitems / ranges}));
 }
 
+// list_splits with the workspace of na sums per target; one wave per item needs none
+static int fit_list_splits(vpm_field f, const DevPlan& dp, int na, int& S)
+{
+    int64_t K = list_splits(dp);
+    const int rc = fit_splits(K, [&](int64_t m) {
+        return m == 1 ? VPM_OK : ensure(f->part, sizeof(double) * na * 64 * (size_t)(dp.nitems * m));
+    });
+    S = (int)K;
+    return rc;
+}
+
 // The source ranges of the k-th of S waves of an item
 __device__ __forceinline__ void take_split(RangeItem& it, int k, int S)
 {
@@ -657,9 +668,8 @@ int launch_p2p_plan(vpm_field f, int kernel, int precision, const DevPlan& dp)
         }
     } else if (dp.wave) {
         const int64_t ni = dp.nitems;
-        const int S = list_splits(dp);
-        if (S > 1)
-            if (int rc = ensure(f->part, sizeof(double) * kAccF32 * 64 * (size_t)(ni * S))) return rc;
+        int S;
+        if (int rc = fit_list_splits(f, dp, kAccF32, S)) return rc;
         double* part = (double*)f->part.p;
         const auto blocks = [](int64_t waves) { return dim3((unsigned)((waves + kBlock / 64 - 1) / (kBlock / 64))); };
         switch (kernel) {
@@ -1375,9 +1385,8 @@ int launch_estr_plan(vpm_field f, int kernel, int precision, int transposed, con
     }
     if (!f64 && dp.wave) {
         const int64_t ni = dp.nitems;
-        const int nsplit = list_splits(dp);
-        if (nsplit > 1)
-            if (int rc = ensure(f->part, sizeof(double) * 6 * 64 * (size_t)(ni * nsplit))) return rc;
+        int nsplit;
+        if (int rc = fit_list_splits(f, dp, 6, nsplit)) return rc;
         double* part = (double*)f->part.p;
         const auto blocks = [](int64_t waves) { return dim3((unsigned)((waves + kBlock / 64 - 1) / (kBlock / 64))); };
         switch (kernel) {

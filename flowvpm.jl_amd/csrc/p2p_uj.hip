@@ -652,12 +652,16 @@ static int launch_uj_split(vpm_field ft, const Staged& T, int64_t nt, const Stag
                            Arena* ar, int64_t kmax)
 {
     const int64_t bt = far_batch(nt, ns);
-    const FarSplit k = far_split(bt, ns, kmax);
+    FarSplit k;
     int rc;
     void *fp, *pp;
-    if ((rc = take_buffer(ft, ft->far, far_scratch_bytes(bt, ns), ar, fp, "far field"))) return rc;
-    const size_t bytes = sizeof(double) * kAccF32 * (size_t)(k.far + k.rest) * (size_t)bt;
-    if ((rc = take_buffer(ft, ft->part, bytes, ar, pp, "partial sums"))) return rc;
+    if ((rc = take_buffer(ft, ft->far, far_scratch_bytes(bt, ns), ar, fp, "far field")) ||
+        (rc = fit_far_split(bt, ns, kmax, k, [&](size_t bytes) {
+             return take_buffer(ft, ft->part, bytes, ar, pp, "partial sums");
+         }))) {
+        if (rc == VPM_ENOMEM) release(ft->far);
+        return rc;
+    }
     double* part = (double*)pp;
     for (int64_t t0 = 0; t0 < nt; t0 += bt) {
         const int64_t n = std::min(bt, nt - t0);
@@ -675,8 +679,11 @@ int launch_uj(vpm_field ft, const Staged& T, int64_t t0, int64_t nt, const Stage
               int64_t s1, int kernel, int precision, bool far, Arena* ar, int64_t kmax)
 {
     if (nt <= 0 || s1 <= s0) return VPM_OK;
-    if (far && t0 == 0 && s0 == 0 && far_applies(kernel, precision, nt, s1))
-        return launch_uj_split(ft, T, nt, S, s1, kernel, ar, kmax);
+    if (far && t0 == 0 && s0 == 0 && far_applies(kernel, precision, nt, s1)) {
+        // where memory holds no split of it, the pair kernel takes all
+        const int rc = launch_uj_split(ft, T, nt, S, s1, kernel, ar, kmax);
+        if (rc != VPM_ENOMEM) return rc;
+    }
     int64_t K, chunk;
     choose_split(nt, s1 - s0, kmax, K, chunk);
     const int acc = precision == VPM_PREC_F64 ? kAccF64 : kAccF32;

@@ -5,20 +5,8 @@
 
 namespace vpm {
 
-// Source splits of the two kernels of a launch.
-struct FarSplit {
-    int64_t far = 1, chunk = 1;   // far kernel: splits, tiles per split
-    int64_t rest = 1;             // rest kernel: splits (every rest-th tile)
-};
-
 // Whether an all-pairs launch is split at all.
 bool far_applies(int kernel, int precision, int64_t nt, int64_t ns);
-// Targets per launch: the words of one launch stay within 256 MiB.
-int64_t far_batch(int64_t nt, int64_t ns);
-// Scratch of one launch (boxes and words).
-size_t far_scratch_bytes(int64_t nt, int64_t ns);
-// kmax > 0 caps each kernel's splits.
-FarSplit far_split(int64_t nt, int64_t ns, int64_t kmax);
 // Partial sums [k.far + k.rest][kAccF32][nt] of sources [0, ns) of S on
 // targets [t0, t0 + nt) of T.
 int launch_uj_far(hipStream_t stream, const Staged& T, int64_t t0, int64_t nt, const Staged& S, int64_t ns, int kernel,

@@ -84,14 +84,6 @@ constexpr double kRsqMean = 1.0 + 3.5e-8;
 // / 1.1e-4, jet 2.8e-5 / 2.6e-5 -> 1.5e-5 / 1.5e-5).
 constexpr int64_t kFarPairs = (int64_t)1 << 28;
 constexpr int64_t kFarMin = 2048;
-// Blocks of a launch.  The far kernel's blocks do equal work per tile; 2,048
-// or 8,192 of them measure the same at N = 65,536, and fewer splits leave
-// fewer partial sums.  The rest kernel's work per wave is uneven (a wave whose
-// targets are scattered reaches most sources), so it has at least 16 splits:
-// 352 ms at 2^20 with 16 or more, 358 with 8, 401 with 2.
-constexpr int64_t kFarBlocks = 2048;
-constexpr int64_t kRestBlocks = 4096;
-constexpr int64_t kRestMin = 16;
 constexpr int kFarThreads = 512;     // threads of a block of 256 targets
 
 // Box of each run of 64 consecutive particles: lo, hi, then the largest
@@ -579,38 +571,6 @@ bool far_applies(int kernel, int precision, int64_t nt, int64_t ns)
     return cheap && precision == VPM_PREC_F32C && nt >= kFarMin && ns >= kFarMin && nt * ns >= kFarPairs;
 }
 
-static int64_t up256(int64_t b) { return (b + 255) & ~(int64_t)255; }
-
-int64_t far_batch(int64_t nt, int64_t ns)
-{
-    const int64_t ntile = (ns + kTile - 1) / kTile;
-    const int64_t most = std::max<int64_t>(1, ((int64_t)64 << 20) / ntile) * kBlock;
-    return std::min(nt, most);
-}
-
-size_t far_scratch_bytes(int64_t nt, int64_t ns)
-{
-    const int64_t nwave = (nt + 63) / 64, ngroup = (ns + 63) / 64;
-    const int64_t nblk = (nt + kBlock - 1) / kBlock, ntile = (ns + kTile - 1) / kTile;
-    return (size_t)(up256(64 * nwave) + up256(64 * ngroup) + up256(4 * nblk * ntile));
-}
-
-FarSplit far_split(int64_t nt, int64_t ns, int64_t kmax)
-{
-    const int64_t nblk = (nt + kBlock - 1) / kBlock, ntile = (ns + kTile - 1) / kTile;
-    const auto cap = [&](int64_t K) {
-        K = std::max<int64_t>(1, K);
-        if (kmax > 0) K = std::min(K, kmax);
-        return std::min(K, ntile);
-    };
-    FarSplit k;
-    k.far = cap(kFarBlocks / nblk);
-    k.chunk = (ntile + k.far - 1) / k.far;
-    k.far = (ntile + k.chunk - 1) / k.chunk;
-    k.rest = cap(std::max<int64_t>(kRestMin, kRestBlocks / nblk));
-    return k;
-}
-
 int launch_uj_far(hipStream_t stream, const Staged& T, int64_t t0, int64_t nt, const Staged& S, int64_t ns, int kernel,
                   const FarSplit& k, void* scratch, double* part)
 {
@@ -618,8 +578,8 @@ int launch_uj_far(hipStream_t stream, const Staged& T, int64_t t0, int64_t nt, c
     const unsigned nblk = (unsigned)((nt + kBlock - 1) / kBlock), ntile = (unsigned)((ns + kTile - 1) / kTile);
     char* p = (char*)scratch;
     double* tbox = (double*)p;
-    double* gbox = (double*)(p + up256(64 * nwave));
-    uint32_t* words = (uint32_t*)(p + up256(64 * nwave) + up256(64 * ngroup));
+    double* gbox = (double*)(p + far_up256(64 * nwave));
+    uint32_t* words = (uint32_t*)(p + far_up256(64 * nwave) + far_up256(64 * ngroup));
     double* rest = part + (size_t)k.far * kAccF32 * (size_t)nt;
     hipLaunchKernelGGL(far_box_kernel, dim3(nblk), dim3(kBlock), 0, stream, T.pos, T.ld, t0, nt, (const float*)nullptr,
                        (const float4*)nullptr, tbox);

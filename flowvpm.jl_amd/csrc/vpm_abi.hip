@@ -72,7 +72,7 @@ int ensure_pinned(DevBuf& b, size_t bytes)
     return VPM_OK;
 }
 
-static void release(DevBuf& b)
+void release(DevBuf& b)
 {
     if (b.p) (void)hipFree(b.p);
     b.p = nullptr;

@@ -9,6 +9,7 @@
 
 #include "../../include/flowvpm_hip.h"
 #include "range_plan.h"
+#include "uj_split.h"
 
 namespace vpm {
 
@@ -26,10 +27,6 @@ constexpr double kConst3 = 0x1.e8ec8a4aeacc4p-3;    // 3/(4*pi)
 constexpr double kConst4 = 0x1.45f306dc9c883p-4;    // 1/(4*pi)
 constexpr double kSqr2 = 0x1.6a09e667f3bcdp+0;      // sqrt(2)
 
-constexpr int kBlock = 256;      // threads per block (4 waves of 64)
-constexpr int kTile = 256;       // sources per LDS tile
-constexpr int kAccF32 = 14;      // U'(3) W'(3) Jhv(8) per target, F32C path
-constexpr int kAccF64 = 12;      // U(3) J(9) per target, F64 path
 // internal precision of the FP64 far-form U/J kernel (vpm_uj_direct with
 // VPM_PREC_F64 and VPM_UJ_F64_FAR)
 constexpr int kPrecF64Far = 2;
@@ -133,6 +130,7 @@ int fail(int status, const std::string& msg);
 int hip_fail(hipError_t e, const char* what);
 // ensure a grow-only buffer holds at least `bytes`
 int ensure(DevBuf& b, size_t bytes);
+void release(DevBuf& b);
 // the same for pinned host memory; the caller has synchronized the field's
 // stream since the buffer's last use as a copy source
 int ensure_pinned(DevBuf& b, size_t bytes);
