@@ -5,6 +5,9 @@
 
 namespace vpm {
 
+// Fewest particles of a field whose time steps take the far kernel.
+constexpr int64_t kFarStepMin = 1 << 16;
+
 // Whether an all-pairs launch is split at all.
 bool far_applies(int kernel, int precision, int64_t nt, int64_t ns);
 // Partial sums [k.far + k.rest][kAccF32][nt] of sources [0, ns) of S on

@@ -70,18 +70,10 @@ constexpr float kSqScale = 4096.f;   // scale of t^2 in the r^2 product
 // v_rsq_f32 is low by 5.8e-9 of its result on [1, 2) and 8.1e-9 on [2, 4)
 // (means weighted by 1/x), so r^-5 by 3.5e-8 wherever r lies.
 constexpr double kRsqMean = 1.0 + 3.5e-8;
-// The far kernel pays from 16,384 particles, in U/J alone, with E_str and in
-// time steps alike.  With every pair on the VALU, and with the far kernel: U/J
-// of the cloud, the jet, the leapfrog rings and a thin ring 0.208 / 0.233,
-// 0.183 / 0.194, 0.223 / 0.259 and 0.182 / 0.198 ms at 12,288 (boxes of 64
-// particles are too large for most pairs to be far), 0.320 / 0.322, 0.291 /
-// 0.301, 0.347 / 0.318 and 0.278 / 0.274 at 16,384, 0.457 / 0.404, 0.415 /
-// 0.355, 0.459 / 0.423 and 0.396 / 0.344 at 20,000; their steps 1.41 / 1.43,
-// 1.30 / 1.33, 1.52 / 1.40 and 1.25 / 1.23 ms at 16,384, 2.03 / 1.77, 1.84 /
-// 1.58, 2.03 / 1.84 and 1.76 / 1.53 at 20,000.  E_str, a sum of differences of
-// J, is the more precise for it (RMS per unit of its scale at 16,384 / 65,536:
-// rings 1.4e-6 / 1.1e-5 -> 4.1e-7 / 4.1e-6, thin ring 5.3e-5 / 1.8e-4 -> 2.9e-5
-// / 1.1e-4, jet 2.8e-5 / 2.6e-5 -> 1.5e-5 / 1.5e-5).
+// The far kernel pays from about 16,384 particles (U/J of the cloud, the jet
+// and the leapfrog rings, with and without it: 0.279 / 0.287, 0.255 / 0.264 and
+// 0.271 / 0.313 ms at 16,384; 0.139 / 0.110 ms for the cloud at 8,192, where
+// boxes of 64 particles are too large for most of their pairs to be far).
 constexpr int64_t kFarPairs = (int64_t)1 << 28;
 constexpr int64_t kFarMin = 2048;
 constexpr int kFarThreads = 512;     // threads of a block of 256 targets

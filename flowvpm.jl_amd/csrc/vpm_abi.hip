@@ -132,7 +132,7 @@ static int sync(vpm_field f)
 }
 
 // UJ_direct body on a locked field (src/FLOWVPM_UJ.jl:21-37)
-static int uj_direct_locked(vpm_field f, const vpm_config* cfg, uint32_t flags)
+static int uj_direct_locked(vpm_field f, const vpm_config* cfg, uint32_t flags, bool step = false)
 {
     int rc;
     const bool far64 = flags & VPM_UJ_F64_FAR;
@@ -142,7 +142,12 @@ static int uj_direct_locked(vpm_field f, const vpm_config* cfg, uint32_t flags)
     if (flags & VPM_UJ_RESET_SFS) if ((rc = launch_reset(f, 1))) return rc;
     const int prec = far64 ? kPrecF64Far : cfg->precision;
     const bool sort = (cfg->precision == VPM_PREC_F32C || far64) && !(flags & VPM_UJ_NO_SORT);
-    const bool far = sort && far_applies(cfg->kernel, prec, f->np, f->np);
+    // The far kernel, where the spatial order makes groups far.  E_str on
+    // smooth fields is a difference of nearly equal J (1e-3 of it is the FP32
+    // rounding of J on thin rings), so a call that returns E_str keeps the
+    // rounding of the VALU kernel; the steps of small fields too.
+    const bool far = sort && far_applies(cfg->kernel, prec, f->np, f->np) &&
+                     (step ? f->np >= kFarStepMin : !(flags & VPM_UJ_SFS));
     const Order order = !sort ? kStorage : far ? kHilbert : kZOrder;
     Staged st;
     if ((rc = stage_field(f, cfg->kernel, prec, order, st))) return rc;
@@ -159,13 +164,13 @@ static int uj_direct_locked(vpm_field f, const vpm_config* cfg, uint32_t flags)
 
 // uj_flags: VPM_UJ_F64_FAR or 0, as the step's own U/J evaluations
 static int sfs_before_locked(vpm_field f, const vpm_config* cfg, double alpha, double minC, double maxC,
-                             uint32_t uj_flags = 0)
+                             uint32_t uj_flags = 0, bool step = false)
 {
     if (minC < 0 || maxC < 0 || minC > maxC)                         // subfilterscale.jl:455-461
         return fail(VPM_EINVAL, "Invalid C bounds");
     int rc;
     if ((rc = launch_scale_sigma(f, alpha, 0))) return rc;
-    if ((rc = uj_direct_locked(f, cfg, VPM_UJ_RESET | VPM_UJ_RESET_SFS | VPM_UJ_SFS | uj_flags))) return rc;
+    if ((rc = uj_direct_locked(f, cfg, VPM_UJ_RESET | VPM_UJ_RESET_SFS | VPM_UJ_SFS | uj_flags, step))) return rc;
     if ((rc = launch_sfs_store_test(f, cfg->transposed))) return rc;
     return launch_scale_sigma(f, alpha, 1);
 }
@@ -623,7 +628,7 @@ static int rk3_step_locked(vpm_field f, vpm_step_config* s, double dt, int32_t r
     const double zeta0 = zeta0_of(cfg->kernel);                    // timeintegration.jl:398
     const bool sfs = s->sfs != 0;
     // the spatial order of the step's U/J evaluations (uj_direct_locked)
-    const Order order = far_applies(cfg->kernel, cfg->precision, f->np, f->np) ? kHilbert : kZOrder;
+    const Order order = far_applies(cfg->kernel, cfg->precision, f->np, f->np) && f->np >= kFarStepMin ? kHilbert : kZOrder;
     int rc;
     bool reset_needed = false, unconverged = false;
     const size_t rec = sizeof(double) * NF * (size_t)f->np;
@@ -645,10 +650,11 @@ static int rk3_step_locked(vpm_field f, vpm_step_config* s, double dt, int32_t r
                               cfg->kernel != VPM_KERNEL_SINGULAR && 1.0 - s->sfs_alpha <= 0.01 &&
                               s->sfs_alpha < 1.0;
         if (sfs && first && !sfs_diff)
-            if ((rc = sfs_before_locked(f, cfg, s->sfs_alpha, s->sfs_minC, s->sfs_maxC, (uint32_t)s->uj_flags)))
+            if ((rc = sfs_before_locked(f, cfg, s->sfs_alpha, s->sfs_minC, s->sfs_maxC, (uint32_t)s->uj_flags,
+                                        true)))
                 return rc;
         const uint32_t fl = VPM_UJ_RESET | (sfs ? (VPM_UJ_RESET_SFS | VPM_UJ_SFS) : 0u) | (uint32_t)s->uj_flags;
-        if ((rc = uj_direct_locked(f, cfg, fl))) return rc;  // :422
+        if ((rc = uj_direct_locked(f, cfg, fl, true))) return rc;  // :422
         if (tape && f->np > 0) {
             hipError_t e = hipMemcpyAsync((char*)tape->rec.p + st * rec, f->P, rec, hipMemcpyDeviceToDevice,
                                           f->stream);
@@ -687,7 +693,7 @@ static int rk3_step_locked(vpm_field f, vpm_step_config* s, double dt, int32_t r
     }
     if (relax_now && s->relax) {                                    // :437-458
         if ((rc = launch_reset(f, 0))) return rc;
-        if ((rc = uj_direct_locked(f, cfg, VPM_UJ_RESET | (uint32_t)s->uj_flags))) return rc;
+        if ((rc = uj_direct_locked(f, cfg, VPM_UJ_RESET | (uint32_t)s->uj_flags, true))) return rc;
         if ((rc = launch_relax(f, s->rlxf, s->relax == 2))) return rc;
     }
     if ((rc = launch_update_uprev(f))) return rc;                   // particlefield.jl:443-455
