@@ -32,7 +32,19 @@ PEAK_FP64 = 78.6e12
 # HBM bytes per U/J launch from two rocprofv3 --pmc runs of this script
 # (FETCH_SIZE scaled by 2.0 and WRITE_SIZE by 1.0, the factors a 256 MiB
 # device copy reads back), keyed by (N, kernel)
-TRAFFIC_BYTES = {(1 << 20, "gaussianerf"): ((3.1774e6 + 1.1093e6) * 2.0 + 1.1469e5 + 1.8350e6) * 1024}
+TRAFFIC_BYTES = {(1 << 20, "gaussianerf"): ((3.1820e6 + 1.1085e6) * 2.0 + 1.1469e5 + 1.8350e6) * 1024}
+# The far kernel's own bound: the issue cycles of a SIMD that the weights of 64
+# pairs take on the VALU (one reciprocal square root of 8.3, three products of
+# 2.6, a packed conversion of 4.6 and a mixed-precision remainder of 4.4, each
+# measured alone), on 1,024 SIMDs at 2.4 GHz, in pairs/s.
+FAR_VALU_CYCLES = 8.3 + 3 * 2.6 + 4.6 + 4.4
+PEAK_FAR_PAIRS = 1024 * 2.4e9 * 64 / FAR_VALU_CYCLES
+
+
+def far_applies(kernel, n):
+    """Whether all-pairs U/J of n particles takes the far field to the matrix
+    cores: far_applies of csrc/uj_far.hip."""
+    return kernel in ("gaussianerf", "gaussian") and n >= 2048 and n * n >= 1 << 28
 
 
 def log(*a):
@@ -550,9 +562,11 @@ def main():
     kms, kcount = f.timing(0)
     k_avg_s = kms / 1e3 / max(kcount, 1)
     value = pairs / (wall / args.steps)
-    achieved = pairs * FLOP_PER_PAIR[kernel] / k_avg_s
-    # the far field of large launches runs on the matrix cores (csrc/uj_far.hip)
-    far = kernel in ("gaussianerf", "gaussian") and n * n >= 1 << 28
+    far = far_applies(kernel, n)
+    if far:
+        achieved, peak, rate = pairs / k_avg_s, PEAK_FAR_PAIRS, "Tpairs/s"
+    else:
+        achieved, peak, rate = pairs * FLOP_PER_PAIR[kernel] / k_avg_s, PEAK_FP32, "TFLOP/s"
     out32 = np.zeros_like(P)
     f.get_particles(out32, rows=(9, 24))
     log("bench: F32C %.1f ms/step, kernel %.1f ms, %.3e pairs/s" % (ms_step, 1e3 * k_avg_s, value))
@@ -566,8 +580,8 @@ def main():
                                                           "accumulation, near pairs FP32 with compensated sums" if far
                                                           else "FP32 pair arithmetic with compensated sums"),
                    "N": n, "kernel": kernel, "pairs_per_step": pairs, "flop_per_pair": FLOP_PER_PAIR[kernel]},
-        "roofline": {"bound": "valu", "achieved": achieved / 1e12, "peak": PEAK_FP32 / 1e12, "unit": "TFLOP/s",
-                     "frac": achieved / PEAK_FP32, "traffic": TRAFFIC_BYTES.get((n, kernel)),
+        "roofline": {"bound": "valu", "achieved": achieved / 1e12, "peak": peak / 1e12, "unit": rate,
+                     "frac": achieved / peak, "traffic": TRAFFIC_BYTES.get((n, kernel)),
                      "kernel": ("uj_far_kernel + uj_rest_kernel<%s>" if far else "uj_f32c_kernel<%s>") % kernel,
                      "avg_launch_ms": 1e3 * k_avg_s,
                      "traffic_source": "profiles/uj_far_gaussianerf_jet_n1048576.md (rocprofv3 FETCH_SIZE x2.0 + "

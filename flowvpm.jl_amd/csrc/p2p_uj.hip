@@ -631,7 +631,8 @@ int64_t split_grain(int64_t nblk, int64_t ns)
 // balance the CUs better than a few long ones: against 2,560 blocks, 32,768
 // run 11-25 % faster from N = 32,768 to 262,144, and at N = 2^20 (K = 8
 // instead of 1) 3-5 % faster; beyond that the gain is flat.  The FP64 partial
-// sums then take at most ~1 GB (K x 14 x 8 B per target).
+// sums then take at most ~1 GB (K x 14 x 8 B per target; the far kernel's
+// launches with at least 17 splits 2 GB, fewer where memory does not hold them).
 void choose_split(int64_t nt, int64_t ns, int64_t kmax, int64_t& K, int64_t& chunk)
 {
     const int64_t nblk = (nt + kBlock - 1) / kBlock;

@@ -5,7 +5,10 @@
 
 namespace vpm {
 
-// Fewest particles of a field whose time steps take the far kernel.
+// Fewest particles of a field whose time steps take the far kernel (the line
+// that keeps a step's results what they are: uj_direct_locked in vpm_abi.hip;
+// it would pay from 18,000: steps of the cloud, the jet, the leapfrog rings and
+// a thin ring 2.03 / 1.84 / 2.03 / 1.76 -> 1.77 / 1.58 / 1.84 / 1.53 ms at 20,000).
 constexpr int64_t kFarStepMin = 1 << 16;
 
 // Whether an all-pairs launch is split at all.

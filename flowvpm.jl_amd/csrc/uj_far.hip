@@ -70,10 +70,15 @@ constexpr float kSqScale = 4096.f;   // scale of t^2 in the r^2 product
 // v_rsq_f32 is low by 5.8e-9 of its result on [1, 2) and 8.1e-9 on [2, 4)
 // (means weighted by 1/x), so r^-5 by 3.5e-8 wherever r lies.
 constexpr double kRsqMean = 1.0 + 3.5e-8;
-// The far kernel pays from about 16,384 particles (U/J of the cloud, the jet
-// and the leapfrog rings, with and without it: 0.279 / 0.287, 0.255 / 0.264 and
-// 0.271 / 0.313 ms at 16,384; 0.139 / 0.110 ms for the cloud at 8,192, where
-// boxes of 64 particles are too large for most of their pairs to be far).
+// The far kernel pays from 16,384 particles.  U/J of the cloud, the jet, the
+// leapfrog rings and a thin ring with every pair on the VALU, and with it: 0.208
+// / 0.233, 0.183 / 0.194, 0.223 / 0.259 and 0.182 / 0.198 ms at 12,288 (boxes
+// of 64 particles are too large for most pairs to be far), 0.320 / 0.322, 0.291
+// / 0.301, 0.347 / 0.318 and 0.278 / 0.274 at 16,384, 0.457 / 0.404, 0.415 /
+// 0.355, 0.459 / 0.423 and 0.396 / 0.344 at 20,000.  Where nearly every pair is
+// near it costs the words and the smaller tiles of the rest kernel: the 65,536
+// cloud with four times its core sizes 6.5 -> 6.9 ms, ten times 6.9 -> 7.2, one
+// of density ~ r^-2 3.8 -> 4.1 (0.38 -> 0.41 at 16,384, 18.3 -> 14.3 at 150,000).
 constexpr int64_t kFarPairs = (int64_t)1 << 28;
 constexpr int64_t kFarMin = 2048;
 constexpr int kFarThreads = 512;     // threads of a block of 256 targets

@@ -142,10 +142,17 @@ static int uj_direct_locked(vpm_field f, const vpm_config* cfg, uint32_t flags, 
     if (flags & VPM_UJ_RESET_SFS) if ((rc = launch_reset(f, 1))) return rc;
     const int prec = far64 ? kPrecF64Far : cfg->precision;
     const bool sort = (cfg->precision == VPM_PREC_F32C || far64) && !(flags & VPM_UJ_NO_SORT);
-    // The far kernel, where the spatial order makes groups far.  E_str on
-    // smooth fields is a difference of nearly equal J (1e-3 of it is the FP32
-    // rounding of J on thin rings), so a call that returns E_str keeps the
-    // rounding of the VALU kernel; the steps of small fields too.
+    // The far kernel, where the spatial order makes groups far, but neither for
+    // calls that return E_str nor in steps below kFarStepMin.  Not for its
+    // precision: E_str, a sum of differences of nearly equal J, is nearer FP64
+    // with the far kernel's J (RMS per unit of its scale at 16,384 / 65,536:
+    // leapfrog rings 1.4e-6 / 1.1e-5 -> 4.1e-7 / 4.1e-6, thin ring 5.3e-5 /
+    // 1.8e-4 -> 2.9e-5 / 1.1e-4, jet 2.8e-5 / 2.6e-5 -> 1.5e-5 / 1.5e-5), nor
+    // for its time (with E_str, 65,536 of them 3.6 -> 2.2 ms).  But J's rounding
+    // is that large a part of what these calls return that another kernel's
+    // moves it by as much: E_str of the jet by 3e-5, of the leapfrog rings by
+    // 6e-5, the strengths of a thin ring after one step by 2e-4 of their size.
+    // Their results stay what they are on the same input.
     const bool far = sort && far_applies(cfg->kernel, prec, f->np, f->np) &&
                      (step ? f->np >= kFarStepMin : !(flags & VPM_UJ_SFS));
     const Order order = !sort ? kStorage : far ? kHilbert : kZOrder;
