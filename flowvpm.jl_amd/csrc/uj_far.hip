@@ -48,8 +48,10 @@
 // 353 (s^2 from LDS 8 ms, the second fold 9).
 // Measured: U/J of the 2^20 jet 709 -> 353 ms (1.55e12 -> 3.1e12 pairs/s), of
 // the 65,536 cloud 3.72 -> 2.50 ms and of the leapfrog rings 3.26 -> 1.80 ms.
-// The far kernel is bound by the VALU: per pair one rsq, three products, two
-// packed conversions of two and a fma_mix.
+// The far kernel is bound by the VALU: per pair one rsq (8.3 cycles of a SIMD
+// for 64 pairs), three products (2.6 each), two packed conversions of two (4.6)
+// and a fma_mix (4.4) are 25 of the 43 cycles that it takes, at 2.1 GHz; the
+// matrix products keep their unit busy a third of the time beside them.
 #include <algorithm>
 #include <cfloat>
 

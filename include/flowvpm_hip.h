@@ -42,7 +42,9 @@ enum { VPM_KERNEL_SINGULAR = 0, VPM_KERNEL_GAUSSIAN = 1,
        VPM_KERNEL_GAUSSIANERF = 2, VPM_KERNEL_WINCKELMANS = 3 };
 
 /* Pair-arithmetic precision.  F32C: FP32 pair arithmetic, compensated
- * per-target sums, results folded into the FP64 state.  F64: the reference's
+ * per-target sums, results folded into the FP64 state (from 2^28 pairs the far
+ * pairs of the Gaussian kernels as products of split FP16 operands with FP32
+ * accumulation, to the precision of FP32 pairs).  F64: the reference's
  * FP64 pair arithmetic (fmm.jl:113-161 with custom_erf64). */
 enum { VPM_PREC_F32C = 0, VPM_PREC_F64 = 1 };
 
@@ -53,8 +55,10 @@ enum { VPM_PREC_F32C = 0, VPM_PREC_F64 = 1 };
  *                  rsqrt per pair and, for Gaussian-erf (q >= 10) and
  *                  Gaussian (q^2 >= 13), the far form F' = r^-3, H'' = r^-5
  *                  where the kernel's g is 1 and q g' is 0 to FP64 rounding;
- *                  near pairs take the reference's g and dg.  It agrees with
- *                  the reference arithmetic to FP64 rounding of the sums.
+ *                  near pairs take FP64 fits of the reduced kernel functions
+ *                  and one exp (Gaussian-erf), a reduced form (Winckelmans) or
+ *                  the reference's g and dg.  It agrees with the reference
+ *                  arithmetic to FP64 rounding of the sums.
  *                  With VPM_UJ_SFS, E_str is evaluated in FP64 over the
  *                  pairs within q = 10 (Gaussian-erf) or q^2 = 14 (Gaussian),
  *                  where zeta has fallen below 2e-22 of zeta(0).
